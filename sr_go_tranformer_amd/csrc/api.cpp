@@ -164,7 +164,7 @@ struct srq_exec {
     int device = 0;
     hipStream_t stream = nullptr;
     int32_t *d_err = nullptr;  // [4] device error words
-    int32_t *h_err = nullptr;  // pinned mirror
+    int32_t *h_err = nullptr;  // pinned: [0..3] mirror of d_err, [4] set by the packers (pack_flag)
     Workspace ws;
     int32_t *h_meta = nullptr;  // pinned metadata staging
     size_t h_meta_n = 0;
@@ -249,6 +249,21 @@ int check_err_flag(srq_exec *e, int code, const char *what) {
         return fail(code, "%s", what);
     }
     return SRQ_OK;
+}
+
+// Error word of a packer call that joins before it returns: pinned host
+// memory, which the kernel writes only when it meets a non-finite value, so
+// that the call ends with one wait and no copy (a copy and its wait were
+// 20 us of a call).  The stream is idle when the word is cleared: every call
+// on an executor that uses it waits for its kernels.
+int32_t *pack_flag(srq_exec *e) {
+    e->h_err[4] = 0;
+    return e->h_err + 4;
+}
+
+int join_pack_flag(srq_exec *e, const char *what) {
+    SRQ_HIP(hipStreamSynchronize(e->stream));
+    return e->h_err[4] ? fail(SRQ_ENONFINITE, "%s", what) : SRQ_OK;
 }
 
 int alloc_weight(srq_model *m, srq_weight &w, int fmt, int64_t rows, int64_t cols) {
@@ -433,7 +448,7 @@ int srq_exec_create(int device, srq_exec **out) {
         return fail(SRQ_EDEVICE, "stream creation failed");
     }
     if (hipMalloc((void **)&e->d_err, sizeof(int32_t) * 4) != hipSuccess ||
-        hipHostMalloc((void **)&e->h_err, sizeof(int32_t) * 4) != hipSuccess) {
+        hipHostMalloc((void **)&e->h_err, sizeof(int32_t) * 8) != hipSuccess) {
         exec_unref(e);
         return fail(SRQ_ENOMEM, "executor allocation failed");
     }
@@ -486,8 +501,8 @@ int srq_pack(srq_exec *e, srq_format fmt, int64_t rows, int64_t cols, const void
     if (fmt != SRQ_Q8 && fmt != SRQ_Q4) return fail(SRQ_EINVAL, "pack format must be Q8 or Q4");
     if (rows < 0 || cols < 0 || dtype < SRQ_SRC_F32 || dtype > SRQ_SRC_F16) return fail(SRQ_EINVAL, "bad shape or dtype");
     DeviceGuard g(e->device);
-    SRQ_CHECK(launch_pack(e->stream, fmt, rows, cols, src, dtype, values, scales, e->d_err));
-    return check_err_flag(e, SRQ_ENONFINITE, "non-finite weight in pack source");
+    SRQ_CHECK(launch_pack(e->stream, fmt, rows, cols, src, dtype, values, scales, pack_flag(e)));
+    return join_pack_flag(e, "non-finite weight in pack source");
 }
 
 int srq_fill_normal(srq_exec *e, float *dst, int64_t count, uint64_t seed, double scale) {
@@ -517,9 +532,10 @@ int srq_weight_create(srq_exec *e, srq_format fmt, int64_t rows, int64_t cols, c
         srq_weight_destroy(w);
         return fail(SRQ_ENOMEM, "weight allocation failed");
     }
-    int rc = fmt == SRQ_F32 ? launch_convert_f32(e->stream, rows * cols, src, dtype, (float *)w->values, e->d_err)
-                            : launch_pack(e->stream, fmt, rows, cols, src, dtype, w->values, w->scales, e->d_err);
-    if (rc == SRQ_OK) rc = check_err_flag(e, SRQ_ENONFINITE, "non-finite weight");
+    int32_t *const flag = pack_flag(e);
+    int rc = fmt == SRQ_F32 ? launch_convert_f32(e->stream, rows * cols, src, dtype, (float *)w->values, flag)
+                            : launch_pack(e->stream, fmt, rows, cols, src, dtype, w->values, w->scales, flag);
+    if (rc == SRQ_OK) rc = join_pack_flag(e, "non-finite weight");
     if (rc != SRQ_OK) {
         srq_weight_destroy(w);
         return rc;

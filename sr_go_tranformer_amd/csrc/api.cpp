@@ -344,6 +344,26 @@ size_t linear_scratch_bytes(const srq_weight &w, int32_t n, int32_t gemm_rows = 
     return n > gemm_rows && gemm_ok(w.fmt, w.cols) ? gemm_scratch_bytes(w.fmt, n, w.rows, w.cols) : 0;
 }
 
+// Workspace for launch_gemm: what it wants (split-K partial sums and, for
+// many rows, the activations' planes), or only what it needs where the
+// larger buffer cannot be had -- no memory, or a stream under capture, in
+// which nothing may be allocated and a call that needs no scratch still runs.
+int ensure_gemm(srq_exec *e, Workspace &ws, int fmt, int32_t n, int64_t rows, int64_t cols) {
+    const size_t wanted = gemm_scratch_wanted(fmt, n, rows, cols);
+    if (wanted <= ws.flags.n) return SRQ_OK;
+    const size_t need = gemm_scratch_bytes(fmt, n, rows, cols);
+    if (wanted > need) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        SRQ_HIP(hipStreamIsCapturing(e->stream, &cap));
+        if (cap == hipStreamCaptureStatusNone) {
+            if (ensure(ws.flags, wanted, e->stream) == SRQ_OK) return SRQ_OK;
+            (void)hipGetLastError();
+            clear_error();
+        }
+    }
+    return ensure(ws.flags, need, e->stream);
+}
+
 // y[n x w.rows] = x . W^T for n rows through the GEMV (chunks of 8) or the
 // MFMA GEMM (n > gemm_rows, K multiple of 32), with optional fused RMSNorm.
 // fixed (non-null): the GEMM's scratch is that caller-provided buffer of
@@ -354,7 +374,7 @@ int run_linear(srq_exec *e, Workspace &ws, const srq_weight &w, const float *x, 
     if (n > gemm_rows && gemm_ok(w.fmt, w.cols) && !norm_w) {
         GemmArgs g{w.fmt, w.values, w.scales, w.rows, w.cols, x, n, y, y_stride, residual, nullptr};
         if (fixed) return launch_gemm(e->stream, g, fixed, fixed_bytes);
-        SRQ_CHECK(ensure(ws.flags, gemm_scratch_bytes(w.fmt, n, w.rows, w.cols), e->stream));
+        SRQ_CHECK(ensure_gemm(e, ws, w.fmt, n, w.rows, w.cols));
         return launch_gemm(e->stream, g, ws.flags.p, ws.flags.n);
     }
     const int nb = gemv_max_rows(w.fmt, w.cols, norm_w != nullptr, 0);
@@ -1239,7 +1259,7 @@ int enqueue_layers(srq_exec *e, Workspace &ws, srq_model *m, srq_pool *pool, int
             // projection wrote it from its reduction.
             if (l == 0) SRQ_CHECK(launch_rmsnorm(e->stream, X, L.n1, N, n, (int32_t)d, c.norm_eps));
             // q/k/v GEMM with bias, RoPE and the KV write in its reduction.
-            SRQ_CHECK(ensure(ws.flags, gemm_scratch_bytes(L.qkv.fmt, n, L.qkv.rows, L.qkv.cols), e->stream));
+            SRQ_CHECK(ensure_gemm(e, ws, L.qkv.fmt, n, L.qkv.rows, L.qkv.cols));
             GemmArgs g{L.qkv.fmt, L.qkv.values, L.qkv.scales, L.qkv.rows, L.qkv.cols, N, n, W2, d + 2 * kd,
                        nullptr, nullptr};
             g.rope = GemmRope{Q, L.bias, (int32_t)d, (int32_t)kd, m->hd, m->cos_t, m->sin_t, meta};
@@ -1262,7 +1282,7 @@ int enqueue_layers(srq_exec *e, Workspace &ws, srq_model *m, srq_pool *pool, int
             SRQ_CHECK(run_linear(e, ws, L.o, A, n, X, d, nullptr, 0.0, X, kStepGemmRows));
         } else {
             // with RMSNorm(X, n2) -> N in its reduction
-            SRQ_CHECK(ensure(ws.flags, gemm_scratch_bytes(L.o.fmt, n, L.o.rows, L.o.cols), e->stream));
+            SRQ_CHECK(ensure_gemm(e, ws, L.o.fmt, n, L.o.rows, L.o.cols));
             GemmArgs g{L.o.fmt, L.o.values, L.o.scales, L.o.rows, L.o.cols, A, n, X, d, X, nullptr};
             g.norm_w = L.n2;
             g.norm_eps = c.norm_eps;
@@ -1290,7 +1310,7 @@ int enqueue_layers(srq_exec *e, Workspace &ws, srq_model *m, srq_pool *pool, int
         } else {
             // gate/up GEMM with SwiGLU in its split-K reduction (W2 is only
             // a temporary when K is not split).
-            SRQ_CHECK(ensure(ws.flags, gemm_scratch_bytes(L.gu.fmt, n, L.gu.rows, L.gu.cols), e->stream));
+            SRQ_CHECK(ensure_gemm(e, ws, L.gu.fmt, n, L.gu.rows, L.gu.cols));
             GemmArgs g{L.gu.fmt, L.gu.values, L.gu.scales, L.gu.rows, L.gu.cols, N, n, W2, 2 * H, nullptr, Hh};
             SRQ_CHECK(launch_gemm(e->stream, g, ws.flags.p, ws.flags.n));
         }
@@ -1299,7 +1319,7 @@ int enqueue_layers(srq_exec *e, Workspace &ws, srq_model *m, srq_pool *pool, int
             SRQ_CHECK(run_linear(e, ws, L.down, Hh, n, X, d, nullptr, 0.0, X, kStepGemmRows));
         } else {
             // with the next layer's RMSNorm(X, n1) -> N in its reduction
-            SRQ_CHECK(ensure(ws.flags, gemm_scratch_bytes(L.down.fmt, n, L.down.rows, L.down.cols), e->stream));
+            SRQ_CHECK(ensure_gemm(e, ws, L.down.fmt, n, L.down.rows, L.down.cols));
             GemmArgs g{L.down.fmt, L.down.values, L.down.scales, L.down.rows, L.down.cols, Hh, n, X, d, X, nullptr};
             g.norm_w = m->L[l + 1].n1;
             g.norm_eps = c.norm_eps;

@@ -28,7 +28,7 @@
 #include <algorithm>
 #include <utility>
 
-#include "srq_internal.h"
+#include "gemm_common.h"
 
 namespace srq {
 namespace {
@@ -36,7 +36,6 @@ namespace {
 constexpr int BN = 128, BK = 32, LDK = BK + 4;
 constexpr int kCUs = 256;          // MI355X compute units
 constexpr int kMinSliceInputs = 256;  // inputs per split-K slice, at least
-typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 template <int FMT>
 __device__ __forceinline__ void load_b(const uint8_t *__restrict__ W, const float *__restrict__ S, int64_t rows,
@@ -134,34 +133,6 @@ __device__ __forceinline__ float store_a(float *As, int tid, const float4 (&a)[A
         amax = fmaxf(amax, fmaxf(fmaxf(fabsf(a[i].x), fabsf(a[i].y)), fmaxf(fabsf(a[i].z), fabsf(a[i].w))));
     }
     return amax;
-}
-
-// linearQ8WideInto / linearQ4WideInto (M:4356-4382, M:4754-4780): output o
-// of row m in FP64, per-block partial sums scaled in FP64, plus residual.
-__device__ __forceinline__ double wide_weight(int fmt, const uint8_t *wrow, int64_t c) {
-    if (fmt == SRQ_Q8) return (double)((const int8_t *)wrow)[c];
-    if (fmt == SRQ_Q4) {
-        uint32_t b = wrow[c >> 1];
-        uint32_t nib = (c & 1) ? (b >> 4) : (b & 15u);
-        return (double)(((int32_t)(nib << 28)) >> 28);
-    }
-    return (double)((const float *)wrow)[c];
-}
-
-__device__ __forceinline__ float wide_output(const GemmArgs &G, int64_t m, int64_t o) {
-    const uint8_t *wrow = (const uint8_t *)G.values + o * row_bytes(G.fmt, G.cols);
-    const float *xr = G.x + m * G.cols;
-    const int64_t groups = groups_of(G.cols);
-    double sum = 0.0;
-    for (int64_t g = 0; g < groups; ++g) {
-        double part = 0.0;
-        const int64_t end = (g + 1) * kBlock < G.cols ? (g + 1) * kBlock : G.cols;
-        for (int64_t j = g * kBlock; j < end; ++j) part += (double)xr[j] * wide_weight(G.fmt, wrow, j);
-        sum += part * (G.fmt == SRQ_F32 ? 1.0 : (double)G.scales[o * groups + g]);
-    }
-    float v = (float)sum;
-    if (G.residual) v = G.residual[m * G.y_stride + o] + v;
-    return v;
 }
 
 // partial == nullptr: one slice covers all K and the tile writes y.
@@ -352,18 +323,7 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const GemmArgs G, cons
 //    planes, row stride 72 bf16 (conflict-free 16-byte reads of 16 rows).
 //    Lane (i, q) reads row i, inputs [16q + 8h, 16q + 8h + 8) for half h:
 //    the same K map as the weights.
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));
 constexpr int XLD = 72;
-
-// Workgroup barrier over LDS only.  __syncthreads() also waits for every
-// global load in flight (vmcnt(0)), which in the block loop below would
-// drain the weight and activation loads issued blocks ahead at every block.
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
 
 template <int TM, int NT = 256>
 struct XTile {
@@ -374,86 +334,6 @@ struct XTile {
     static constexpr int PLANE = BM * XLD;    // bf16 per plane
     static_assert(FPT >= 4, "at least one float4 per thread");
 };
-
-__device__ __forceinline__ uint32_t pk_hi16(float lo, float hi) {
-    return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
-}
-
-// One lane's 16 codes of a block: Q8 16 bytes, Q4 8 bytes.
-template <int FMT>
-struct XRaw {
-    typedef uint32_t type __attribute__((ext_vector_type(FMT == SRQ_Q8 ? 4 : 2)));
-};
-
-template <int FMT>
-__device__ __forceinline__ void xload_b(const uint8_t *__restrict__ W, const float *__restrict__ S, int64_t rows,
-                                        int64_t cols, int64_t groups, int64_t row, int64_t g, int q,
-                                        typename XRaw<FMT>::type &raw, float &scale) {
-    typedef typename XRaw<FMT>::type R;
-    if (row < rows) {
-        if constexpr (FMT == SRQ_Q8)
-            raw = *(const R *)(W + row * cols + g * kBlock + 16 * q);
-        else
-            raw = *(const R *)(W + row * (cols / 2) + g * (kBlock / 2) + 8 * q);
-        scale = S[row * groups + g];
-    } else {
-        raw = R{};
-        scale = 0.0f;
-    }
-}
-
-// Codes of one lane's block slice -> the two bf16x8 MFMA operands.
-template <int FMT>
-__device__ __forceinline__ void xcodes(const typename XRaw<FMT>::type raw, bf16x8 &h0, bf16x8 &h1) {
-    u32x4v p0, p1;
-    if constexpr (FMT == SRQ_Q8) {
-#pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            const uint32_t d = raw[w];
-            const float c0 = (float)(int32_t)(int8_t)d, c1 = (float)(int32_t)(int8_t)(d >> 8);
-            const float c2 = (float)(int32_t)(int8_t)(d >> 16), c3 = (float)((int32_t)d >> 24);
-            const uint32_t a = pk_hi16(c0, c1), b = pk_hi16(c2, c3);
-            if (w < 2) {
-                p0[2 * w] = a;
-                p0[2 * w + 1] = b;
-            } else {
-                p1[2 * w - 4] = a;
-                p1[2 * w - 3] = b;
-            }
-        }
-    } else {
-        // code/16 (exact in bf16), one SDWA convert per nibble; the block's
-        // scale carries the factor 16 back (SRQ_CONVERT), so the product
-        // block * scale is unchanged bit for bit
-#pragma unroll
-        for (int w = 0; w < 2; ++w) {
-            const uint32_t d = raw[w], h = d >> 4;
-            u32x4v &p = w == 0 ? p0 : p1;
-            p[0] = pk_hi16(nib16<0>(d), nib16<0>(h));
-            p[1] = pk_hi16(nib16<1>(d), nib16<1>(h));
-            p[2] = pk_hi16(nib16<2>(d), nib16<2>(h));
-            p[3] = pk_hi16(nib16<3>(d), nib16<3>(h));
-        }
-    }
-    h0 = __builtin_bit_cast(bf16x8, p0);
-    h1 = __builtin_bit_cast(bf16x8, p1);
-}
-
-template <int TM>
-__device__ __forceinline__ void xload_a(const float *__restrict__ X, int32_t n, int64_t cols, int64_t m0, int64_t g,
-                                        int tid, float4 (&a)[XTile<TM>::NV]) {
-    constexpr int FPT = XTile<TM>::FPT, TPR = XTile<TM>::TPR, NV = XTile<TM>::NV;
-    const int r = tid / TPR, c = (tid % TPR) * FPT;
-    const int64_t m = m0 + r;
-    if (m < n) {
-        const float4 *p = (const float4 *)(X + m * cols + g * kBlock + c);
-#pragma unroll
-        for (int i = 0; i < NV; ++i) a[i] = p[i];
-    } else {
-#pragma unroll
-        for (int i = 0; i < NV; ++i) a[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-    }
-}
 
 // Splits the staged floats into the hi / mid / lo planes; returns max |x|.
 template <int TM, int NT = 256>
@@ -1349,6 +1229,35 @@ size_t gemm_scratch_bytes(int fmt, int32_t n, int64_t rows, int64_t cols) {
     return (size_t)p.slices * (size_t)n * ((size_t)rows + 1) * 4;
 }
 
+// Whether a call of n rows takes the tall tiles (gemm_tall.hip), given scratch
+// for its planes.  They cost one more launch (about 4 us with its gap).
+// Q4, whose 64-row tiles here convert more per MFMA, gains from 33 rows on
+// (28672 x 4096 at 40 rows 90 -> 57 us, 512 x 512 19.7 -> 14.6 us).  Q8 gains
+// where the MFMAs outweigh the launch: 28672 x 4096 at 96 / 160 rows 101 -> 94
+// / 155 -> 115 us, 3072 x 3072 at 128 / 160 rows 21.2 -> 22.2 / 28.9 -> 28.1,
+// 5120 x 3072 at 128 / 160 rows 26.1 -> 27.6 / 36.0 -> 34.2; and not at up
+// to 64 rows of an unsplit matrix (128256 x 2048 at 40 rows 118 -> 125 us).
+static bool tall_ok(const GemmPlan &p, int fmt, int32_t n, int64_t rows, int64_t cols) {
+    if (!p.x3 || n <= 32 || cols % (4 * kBlock) || cols > kTallMaxCols) return false;
+    if (fmt == SRQ_Q4) return true;
+    const double macs = (double)n * (double)rows * (double)cols;
+    if (p.slices == 1 && n <= 64) return false;
+    return macs >= 3.2e9 || (n > 128 && macs >= 1.4e9);
+}
+
+// Layout: partial sums, their wide-row flags, then (256-aligned) the tall
+// tiles' flags and planes.
+static size_t tall_offset(size_t need) { return (need + 255) / 256 * 256; }
+
+size_t gemm_scratch_wanted(int fmt, int32_t n, int64_t rows, int64_t cols) {
+    const size_t need = gemm_scratch_bytes(fmt, n, rows, cols);
+    if (n <= 0 || rows <= 0 || !gemm_ok(fmt, cols)) return need;
+    const GemmPlan p = plan_gemm(fmt, n, rows, cols);
+    if (!tall_ok(p, fmt, n, rows, cols)) return need;
+    const TallPlan t = tall_plan(n, rows, p.slices);
+    return tall_offset(need + (p.slices == 1 ? (size_t)n * 4 : 0)) + tall_plane_bytes(t, n, cols);
+}
+
 int launch_gemm(hipStream_t s, const GemmArgs &a, void *scratch, size_t scratch_bytes) {
     if (a.n <= 0 || a.rows <= 0) return SRQ_OK;
     if (!gemm_ok(a.fmt, a.cols)) return fail(SRQ_EINVAL, "gemm: cols=%lld not a multiple of %d", (long long)a.cols, BK);
@@ -1370,12 +1279,20 @@ int launch_gemm(hipStream_t s, const GemmArgs &a, void *scratch, size_t scratch_
                      a.rope.dim % a.rope.head_dim || a.rope.kvdim % a.rope.head_dim ||
                      a.rows != (int64_t)a.rope.dim + 2 * (int64_t)a.rope.kvdim || a.y_stride != a.rows))
         return fail(SRQ_EINVAL, "gemm: RoPE/KV output needs rows = dim + 2*kvdim in whole heads and no other epilogue");
-    if (p.bm == 16)
+    if (tall_ok(p, a.fmt, a.n, a.rows, a.cols) && scratch &&
+        scratch_bytes >= gemm_scratch_wanted(a.fmt, a.n, a.rows, a.cols)) {
+        const size_t need = gemm_scratch_bytes(a.fmt, a.n, a.rows, a.cols);
+        const size_t off = tall_offset(need + (p.slices == 1 ? (size_t)a.n * 4 : 0));
+        if (!wflags) wflags = (int32_t *)scratch;
+        SRQ_CHECK(launch_gemm_tall(s, a, tall_plan(a.n, a.rows, p.slices), (uint8_t *)scratch + off, partial, wflags,
+                                   p.slices, p.kper));
+    } else if (p.bm == 16) {
         launch_fmt<16>(s, a, p, partial, wflags);  // bf16 kernel only (plan_gemm)
-    else if (p.bm == 32)
+    } else if (p.bm == 32) {
         launch_fmt<32>(s, a, p, partial, wflags);
-    else
+    } else {
         launch_fmt<64>(s, a, p, partial, wflags);
+    }
     SRQ_HIP(hipGetLastError());
     if (a.rope.q) {
         if (p.slices > 1) {

@@ -163,6 +163,10 @@ struct GemmArgs {
 // memory for split-K partial sums (0: none needed).
 int launch_gemm(hipStream_t s, const GemmArgs &a, void *scratch, size_t scratch_bytes);
 size_t gemm_scratch_bytes(int fmt, int32_t n, int64_t rows, int64_t cols);
+// With this much scratch a call of many rows also keeps its activations'
+// split planes there (gemm_tall.hip); with less it runs the smaller tiles.
+// Either way the results have the same bits.
+size_t gemm_scratch_wanted(int fmt, int32_t n, int64_t rows, int64_t cols);
 bool gemm_ok(int fmt, int64_t cols);
 
 // ------------------------------------------------------------------ glue

@@ -1482,34 +1482,39 @@ extern "C" int srq_sample(srq_exec *e, const float *logits, int32_t rows, const 
     DeviceGuard g(e->device);
     Workspace &ws = e->ws;
     const size_t hist_words = history ? (size_t)rows * history_stride : 0;
-    // [rng: 2*rows][ids: rows][blocked: rows][history_len: rows][row_ids: rows][history]
-    const size_t words = (size_t)rows * 6 + hist_words;
+    // [rng: 2*rows][blocked: rows][history_len: rows][row_ids: rows], then
+    // on the device the history, in the pinned buffer the results
+    // [ids: rows][errors: rows] (the advanced states replace rng there)
+    const size_t words = (size_t)rows * 5 + hist_words;
     SRQ_CHECK(ensure(ws.SMP, words * 4, e->stream));
     SRQ_CHECK(ensure(ws.SMPS, sample_scratch_bytes(rows, vocab), e->stream));
     int32_t *d = as<int32_t>(ws.SMP);
     uint64_t *d_rng = (uint64_t *)d;
-    int32_t *d_ids = d + 2 * rows, *d_blk = d + 3 * rows, *d_hl = d + 4 * rows, *d_rows = d + 5 * rows;
-    int32_t *d_hist = d + 6 * rows;
+    int32_t *d_blk = d + 2 * rows, *d_hl = d + 3 * rows, *d_rows = d + 4 * rows;
+    int32_t *d_hist = d + 5 * rows;
     // The per-row words go through a pinned staging buffer of their own (a
     // queued step may still be copying the metadata buffer; the previous
-    // sampling call ended synchronised) as one copy each way: copies from
-    // pageable memory would each stage and wait on their own.
-    if ((size_t)rows * 6 > e->h_smp_n) {
+    // sampling call ended synchronised) as one copy: copies from pageable
+    // memory would each stage and wait on their own.  The kernel writes its
+    // results back into that buffer (two copies back cost 10 us a call).
+    if ((size_t)rows * 7 > e->h_smp_n) {
         if (e->h_smp) (void)hipHostFree(e->h_smp);
         e->h_smp = nullptr;
         e->h_smp_n = 0;
-        const size_t want = std::max<size_t>((size_t)rows * 6, 1536);
+        const size_t want = std::max<size_t>((size_t)rows * 7, 1536);
         if (hipHostMalloc((void **)&e->h_smp, want * 4) != hipSuccess) return fail(SRQ_ENOMEM, "pinned allocation failed");
         e->h_smp_n = want;
     }
     int32_t *h = e->h_smp;
     std::memcpy(h, rng_state, (size_t)rows * 8);
     for (int32_t r = 0; r < rows; ++r) {
-        h[3 * rows + r] = blocked ? blocked[r] : 0;
-        h[4 * rows + r] = history ? history_len[r] : 0;
-        h[5 * rows + r] = row_ids ? row_ids[r] : 0;
+        h[2 * rows + r] = blocked ? blocked[r] : 0;
+        h[3 * rows + r] = history ? history_len[r] : 0;
+        h[4 * rows + r] = row_ids ? row_ids[r] : 0;
+        h[5 * rows + r] = 0;
+        h[6 * rows + r] = 0;
     }
-    SRQ_HIP(hipMemcpyAsync(d, h, (size_t)rows * 6 * 4, hipMemcpyHostToDevice, e->stream));
+    SRQ_HIP(hipMemcpyAsync(d, h, (size_t)rows * 5 * 4, hipMemcpyHostToDevice, e->stream));
     if (hist_words) SRQ_HIP(hipMemcpyAsync(d_hist, history, hist_words * 4, hipMemcpyHostToDevice, e->stream));
     SampleArgs a{};
     a.logits = logits;
@@ -1525,19 +1530,17 @@ extern "C" int srq_sample(srq_exec *e, const float *logits, int32_t rows, const 
     a.history_stride = history_stride;
     a.blocked = blocked ? d_blk : nullptr;
     a.rng = d_rng;
-    a.ids = d_ids;
-    a.err = e->d_err;
-    SRQ_CHECK(launch_sample(e->stream, a, ws.SMPS.p));
-    // [rng: 2*rows][ids: rows] back in one copy
-    SRQ_HIP(hipMemcpyAsync(h, d, (size_t)rows * 3 * 4, hipMemcpyDeviceToHost, e->stream));
-    SRQ_HIP(hipMemcpyAsync(e->h_err, e->d_err, sizeof(int32_t) * 4, hipMemcpyDeviceToHost, e->stream));
-    SRQ_HIP(hipStreamSynchronize(e->stream));
+    a.rng_out = (uint64_t *)h;
+    a.ids = h + 5 * rows;
+    a.err = h + 6 * rows;
+    const int rc = launch_sample(e->stream, a, ws.SMPS.p);
+    SRQ_HIP(hipStreamSynchronize(e->stream));  // also before h is written again
+    SRQ_CHECK(rc);
     std::memcpy(rng_state, h, (size_t)rows * 8);
-    std::memcpy(ids, h + 2 * rows, (size_t)rows * 4);
-    const int32_t err = e->h_err[0];
+    std::memcpy(ids, h + 5 * rows, (size_t)rows * 4);
+    int32_t err = 0;
+    for (int32_t r = 0; r < rows; ++r) err |= h[6 * rows + r];
     if (err) {
-        SRQ_HIP(hipMemsetAsync(e->d_err, 0, sizeof(int32_t) * 4, e->stream));
-        SRQ_HIP(hipStreamSynchronize(e->stream));
         if (err & 1) return fail(SRQ_ENONFINITE, "non-finite logits");
         if (err & 2) return fail(SRQ_EINVAL, "no candidate token");
         return fail(SRQ_EINVAL, "sampling selection limit exceeded (more than 2048 equal-ranked candidates)");

@@ -21,19 +21,29 @@
 // reference sums f64 probabilities in sorted order; the two agree except
 // when a cut falls within ~1e-12 of a candidate boundary.
 //
-// Three launches.  The first two split each row into chunks, one 256-thread
+// Three launches.  The first two split each row into chunks, one 1024-thread
 // workgroup per (chunk, row): sample_range_kernel finds a chunk's range,
 // candidate count and first maximum; sample_mass_kernel combines the
-// chunks' ranges and writes the chunk's total integer mass and its
-// first-level histogram (2048 buckets over [vmin, vmax]).  sample_kernel,
-// one 1024-thread workgroup per row, adds the chunks' results (exact
-// integer sums, order-free maxima) and makes the cuts: one pass over the
-// row per cut gathers its bucket (more only when a bucket holds over 2048
-// candidates).  The first-level histogram serves all three cuts: every cut
-// is a prefix of the candidate order whose target lies within the prefix
-// kept so far, so the buckets before the one holding it are kept whole and
-// the unfiltered histogram finds the same bucket.  A candidate's mass is
-// recomputed where it is needed (it is a pure function of its value).
+// chunks' ranges and writes the chunk's total integer mass, its first-level
+// histogram (2048 buckets over [vmin, vmax]) and its ids in bucket order.
+// sample_kernel, one 1024-thread workgroup per row, adds the chunks' results
+// (exact integer sums, order-free maxima) and makes the cuts: one pass over
+// the row per cut only when its bucket holds over 2048 candidates.  The
+// first-level histogram serves all three cuts: every cut is a prefix of the
+// candidate order whose target lies within the prefix kept so far, so the
+// buckets before the one holding it are kept whole and the unfiltered
+// histogram finds the same bucket.  A candidate's mass is recomputed where
+// it is needed (it is a pure function of its value).
+//
+// What bounds it: dependent rounds (loads, barriers) in the row kernel, f64
+// exp and LDS atomics in the mass kernel.  About one chunk workgroup per CU,
+// each of 16 waves: two of four waves left the SIMDs waiting and wrote the
+// histograms twice as often; counts and starts share a word, and the listed
+// ids are 16-bit (33 -> 15 MB written at 32 rows of 128256 ids).  The mass of
+// top_k's candidates comes from the cut's running totals, not from a pass
+// over the row.  32 rows x 128256 ids, T 0.8, top-p 0.9, per call 80 -> 62 us
+// (range 10.2 -> 9.4, masses 22.1 -> 18.6, cuts 26.9 -> 16.9, two copies back
+// to the host gone); with top-k 40 and a penalty the cuts took 100 us, now 36.
 #include <algorithm>
 #include <cfloat>
 #include <climits>
@@ -44,23 +54,23 @@ namespace srq {
 namespace {
 
 constexpr int kST = 1024;      // threads of the row kernel
-constexpr int kCT = 256;       // threads of a chunk kernel
+constexpr int kCT = 1024;      // threads of a chunk kernel
 constexpr int kBuckets = 2048;
 constexpr int kList = 2048;    // candidates of one bucket sorted in LDS
 constexpr int kLevels = 4;     // bucket refinements before giving up
 constexpr int kMaxChunks = 64; // chunks per row (one wave scans their shares)
-constexpr int kChunkMax = 8192; // ids per chunk, at most
+constexpr int kChunkMax = 16384; // ids per chunk, at most
 constexpr int kRankSort = 128;  // gathered candidates sorted by rank, at most (8 threads each)
 constexpr double kFix = 17592186044416.0;  // 2^44: mass of probability 1
 // Device scratch of one launch group (ranges, histograms, ids in bucket
-// order: about 1 MiB per row of a 128256-id vocabulary); calls with more
-// rows run in groups that fit it.
-constexpr size_t kSampleScratchMax = (size_t)64 << 20;
+// order: about 450 KiB per row of a 128256-id vocabulary sampled with 31
+// others); calls with more rows run in groups that fit it.
+constexpr size_t kSampleScratchMax = (size_t)32 << 20;
 // The scans give each thread two buckets / two sorted candidates.
 static_assert(kBuckets == 2 * kST && kList == 2 * kST, "two entries per thread");
 static_assert(8 * kRankSort <= kST, "8 threads per ranked candidate");
 static_assert(kMaxChunks <= 64, "one wave combines a row's chunks");
-static_assert(kChunkMax % 256 == 0 && kChunkMax <= 65536, "a chunk in registers, 16-bit ids in a chunk");
+static_assert(kChunkMax % kCT == 0 && kChunkMax < 65536, "a chunk in registers, 16-bit ids and counts in a chunk");
 
 struct Cand {  // a position in candidate order; id INT_MAX = past every candidate
     double v;
@@ -74,8 +84,6 @@ __device__ __forceinline__ bool before(double va, int ia, double vb, int ib) {
 struct SampleLds {
     uint32_t hcount[kBuckets];
     unsigned long long hmass[kBuckets];
-    uint32_t h0count[kBuckets];           // first-level histogram over [vmin, vmax]
-    unsigned long long h0mass[kBuckets];
     double lv[kList];
     int li[kList];
     unsigned long long lp[kList];
@@ -87,9 +95,12 @@ struct SampleLds {
     uint32_t cstart[kMaxChunks + 1];  // level-0 gather: running counts of the chunks' shares
     uint32_t coff[kMaxChunks];        //   and each share's offset in its chunk's bucket order
     int bucket;            // chosen bucket
-    unsigned long long above;
+    uint32_t bucket_n;     //   and its candidates
+    unsigned long long above;   // running count/mass before the bucket
+    unsigned long long mabove;  // running mass before the bucket
     Cand cut;
-    unsigned long long cum;  // running count/mass through the cut
+    unsigned long long cum;   // running count/mass through the cut
+    unsigned long long mcum;  // CUT_COUNT: running mass through the cut
     int found;
 };
 
@@ -117,21 +128,6 @@ __device__ __forceinline__ unsigned long long block_sum(unsigned long long v, Sa
     __syncthreads();
     unsigned long long r = 0;
     for (int w = 0; w < kST / 64; ++w) r += s.red_u[w];
-    __syncthreads();
-    return r;
-}
-// First candidate in order among (v, id) pairs: the largest v, lowest id.
-__device__ __forceinline__ Cand block_first(Cand c, SampleLds &s) {
-    for (int o = 32; o > 0; o >>= 1) {
-        const double ov = __shfl_xor(c.v, o, 64);
-        const int oi = __shfl_xor(c.id, o, 64);
-        if (before(ov, oi, c.v, c.id)) c.v = ov, c.id = oi;
-    }
-    if ((threadIdx.x & 63) == 0) s.red_d[threadIdx.x >> 6] = c.v, s.red_i[threadIdx.x >> 6] = c.id;
-    __syncthreads();
-    Cand r{s.red_d[0], s.red_i[0]};
-    for (int w = 1; w < kST / 64; ++w)
-        if (before(s.red_d[w], s.red_i[w], r.v, r.id)) r.v = s.red_d[w], r.id = s.red_i[w];
     __syncthreads();
     return r;
 }
@@ -232,27 +228,33 @@ __device__ __forceinline__ T wg_reduce(T v, T *red, Op op) {
 }
 
 struct ChunkRed {
-    double d[kCT / 64];
+    double d[kCT / 64], d1[kCT / 64], d2[kCT / 64];
     unsigned long long u[kCT / 64];
-    int i[kCT / 64];
+    int i[kCT / 64], i1[kCT / 64], i2[kCT / 64];
 };
 
-__device__ __forceinline__ Cand wg_first(Cand c, ChunkRed &r) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        const double ov = __shfl_xor(c.v, o, 64);
-        const int oi = __shfl_xor(c.id, o, 64);
-        if (before(ov, oi, c.v, c.id)) c.v = ov, c.id = oi;
+// exp((v - vmax) / T) * 2^44 rounded, the quotient without a division per
+// value: y = RN(1/T), then two residual steps.  The first makes q faithful, the
+// second correctly rounds it (Markstein: a faithful q, an exact residual
+// and a correctly rounded reciprocal).  Temperatures far from 1 divide.
+struct MassOf {
+    double vmax, T, y;
+    bool fast;
+    __device__ MassOf(double vmax_, double T_) : vmax(vmax_), T(T_), y(1.0 / T_), fast(T_ > 0x1p-400 && T_ < 0x1p400) {}
+    __device__ __forceinline__ unsigned long long operator()(double v) const {
+        const double a = v - vmax;
+        double q;
+        if (fast) {
+            q = a * y;
+            q = __builtin_fma(__builtin_fma(-T, q, a), y, q);
+            q = __builtin_fma(__builtin_fma(-T, q, a), y, q);
+        } else {
+            q = a / T;
+        }
+        if (q < -32.0) return 0;  // exp(-32) * 2^44 < 1/2
+        return (unsigned long long)(exp(q) * kFix + 0.5);
     }
-    if ((threadIdx.x & 63) == 0) r.d[threadIdx.x >> 6] = c.v, r.i[threadIdx.x >> 6] = c.id;
-    __syncthreads();
-    Cand b{r.d[0], r.i[0]};
-#pragma unroll
-    for (int w = 1; w < kCT / 64; ++w)
-        if (before(r.d[w], r.i[w], b.v, b.id)) b.v = r.d[w], b.id = r.i[w];
-    __syncthreads();
-    return b;
-}
+};
 
 constexpr int kCE = kChunkMax / kCT;  // ids of a chunk per thread
 
@@ -277,7 +279,11 @@ __global__ __launch_bounds__(kCT) void sample_range_kernel(const SampleArgs A) {
     load_chunk(lg, c0, c1, x);
     const int blocked = A.blocked ? A.blocked[row] : -1;
     if (A.repeat_penalty != 1.0) seen_bits(A, row, c0, (A.chunk_len + 31) / 32, seen, kCT);
-    int bad = 0, cnt = 0;
+    // In FP32 (the conversion to f64 is exact and monotone), the ids of the
+    // history apart, whose values the penalty makes f64.  A thread's ids
+    // ascend, so `>` keeps the first maximum.
+    int bad = 0, cnt = 0, id32 = INT_MAX;
+    float mx = -INFINITY, mn = INFINITY;
     double vmax = -DBL_MAX, vmin = DBL_MAX;
     Cand best{-DBL_MAX, INT_MAX};
 #pragma unroll
@@ -286,22 +292,52 @@ __global__ __launch_bounds__(kCT) void sample_range_kernel(const SampleArgs A) {
         if (i >= c1) continue;
         bad |= !isfinite(x[k]);
         if (i == blocked) continue;
-        const double v = penalised(A, seen, c0, i, x[k]);
-        vmax = fmax(vmax, v);
-        vmin = fmin(vmin, v);
         ++cnt;
-        if (before(v, i, best.v, best.id)) best.v = v, best.id = i;
+        if (A.repeat_penalty != 1.0 && ((seen[(i - c0) >> 5] >> ((i - c0) & 31)) & 1u)) {
+            const double v = penalised(A, seen, c0, i, x[k]);
+            vmax = fmax(vmax, v);
+            vmin = fmin(vmin, v);
+            if (before(v, i, best.v, best.id)) best.v = v, best.id = i;
+            continue;
+        }
+        if (x[k] > mx) mx = x[k], id32 = i;
+        mn = fminf(mn, x[k]);
     }
-    auto add = [](unsigned long long a, unsigned long long b) { return a + b; };
-    // bad flags in the low word, counts in the high one (at most 2^31 ids)
-    const unsigned long long bc = wg_reduce<kCT>((unsigned long long)bad + ((unsigned long long)cnt << 32), red.u, add);
-    vmax = wg_reduce<kCT>(vmax, red.d, [](double a, double b) { return fmax(a, b); });
-    vmin = wg_reduce<kCT>(vmin, red.d, [](double a, double b) { return fmin(a, b); });
-    best = wg_first(best, red);
+    if (id32 != INT_MAX) {
+        vmax = fmax(vmax, (double)mx);
+        vmin = fmin(vmin, (double)mn);
+        if (before((double)mx, id32, best.v, best.id)) best.v = (double)mx, best.id = id32;
+    }
+    // waves, then wave 0 over the waves' results
+#pragma unroll
+    for (int round = 0; round < 2; ++round) {
+        const int span = round ? kCT / 64 : 64;
+#pragma unroll
+        for (int o = span / 2; o > 0; o >>= 1) {
+            bad |= __shfl_xor(bad, o, 64);
+            cnt += __shfl_xor(cnt, o, 64);
+            vmax = fmax(vmax, __shfl_xor(vmax, o, 64));
+            vmin = fmin(vmin, __shfl_xor(vmin, o, 64));
+            const double ov = __shfl_xor(best.v, o, 64);
+            const int oi = __shfl_xor(best.id, o, 64);
+            if (before(ov, oi, best.v, best.id)) best.v = ov, best.id = oi;
+        }
+        if (round) break;
+        if ((tid & 63) == 0) {
+            const int w = tid >> 6;
+            red.d[w] = vmax, red.d1[w] = vmin, red.d2[w] = best.v;
+            red.i[w] = bad, red.i1[w] = cnt, red.i2[w] = best.id;
+        }
+        __syncthreads();
+        if (tid >= 64) return;
+        const int w = tid & (kCT / 64 - 1);
+        vmax = red.d[w], vmin = red.d1[w], best.v = red.d2[w];
+        bad = red.i[w], cnt = red.i1[w], best.id = red.i2[w];
+    }
     if (tid == 0) {
         SampleRange &o = A.range[(int64_t)row * A.chunks + c];
         o.vmax = vmax, o.vmin = vmin, o.best_v = best.v;
-        o.best_id = best.id, o.cnt = (int)(bc >> 32), o.bad = (bc & 0xffffffffull) != 0;
+        o.best_id = best.id, o.cnt = cnt, o.bad = bad != 0;
     }
 }
 
@@ -348,13 +384,14 @@ __global__ __launch_bounds__(kCT) void sample_mass_kernel(const SampleArgs A) {
     row_range(A, row, red, bad, cnt, vmax, vmin);
     if (bad || cnt == 0) return;  // sample_kernel reports the row
     const int blocked = A.blocked ? A.blocked[row] : -1;
-    const double T = A.temperature;
+    const MassOf mass_of(vmax, A.temperature);
     for (int b = tid; b < kBuckets; b += kCT) hcount[b] = 0, hmass[b] = 0;
     if (A.repeat_penalty != 1.0) seen_bits(A, row, c0, (A.chunk_len + 31) / 32, seen, kCT);
     __syncthreads();
     const double scale0 = vmax > vmin ? (double)kBuckets / (vmax - vmin) : 0.0;
     unsigned long long total = 0;
-    // each id's bucket (-1: no candidate) stays in registers for the listing
+    // each id's bucket and its place there (-1: no candidate) stay in
+    // registers for the listing
     int bk[kCE];
 #pragma unroll
     for (int k = 0; k < kCE; ++k) {
@@ -362,20 +399,19 @@ __global__ __launch_bounds__(kCT) void sample_mass_kernel(const SampleArgs A) {
         bk[k] = -1;
         if (i >= c1 || i == blocked) continue;
         const double v = penalised(A, seen, c0, i, x[k]);
-        const unsigned long long m = (unsigned long long)(exp((v - vmax) / T) * kFix + 0.5);
+        const unsigned long long m = mass_of(v);
         total += m;
         const int b = bucket_of(v, vmin, scale0);
-        bk[k] = b;
-        atomicAdd(&hcount[b], 1u);
-        atomicAdd(&hmass[b], m);
+        bk[k] = b | (int)(atomicAdd(&hcount[b], 1u) * kBuckets);
+        if (m) atomicAdd(&hmass[b], m);
     }
     total = wg_reduce<kCT>(total, red.u, [](unsigned long long x, unsigned long long y) { return x + y; });
     const int64_t h = ((int64_t)row * A.chunks + c) * kBuckets;
-    for (int b = tid; b < kBuckets; b += kCT) A.hcount[h + b] = hcount[b], A.hmass[h + b] = hmass[b];
+    for (int b = tid; b < kBuckets; b += kCT) A.hmass[h + b] = hmass[b];
     if (tid == 0) A.range[(int64_t)row * A.chunks + c].total = total;
 
     // Bucket offsets (exclusive running counts; thread t owns buckets
-    // 8t .. 8t+7), then the chunk's candidate ids listed in bucket order
+    // 2t and 2t+1), then the chunk's candidate ids listed in bucket order
     // (within a bucket in any order: the cuts sort what they gather).
     constexpr int BPT = kBuckets / kCT;
     uint32_t own[BPT], sum = 0;
@@ -395,17 +431,17 @@ __global__ __launch_bounds__(kCT) void sample_mass_kernel(const SampleArgs A) {
     for (int w = 0; w < kCT / 64; ++w) cnt_c += red.i[w];
 #pragma unroll
     for (int k = 0; k < BPT; ++k) {
-        hcount[BPT * tid + k] = start;  // now the bucket's next free slot
-        A.hoff[h + BPT * tid + k] = start;
+        hcount[BPT * tid + k] = start;  // now the bucket's start
+        A.hcount[h + BPT * tid + k] = own[k] | (start << 16);
         start += own[k];
     }
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < kCE; ++k)
-        if (bk[k] >= 0) lorder[atomicAdd(&hcount[bk[k]], 1u)] = (uint16_t)(k * kCT + tid);
+        if (bk[k] >= 0) lorder[hcount[bk[k] & (kBuckets - 1)] + (uint32_t)(bk[k] / kBuckets)] = (uint16_t)(k * kCT + tid);
     __syncthreads();
-    int32_t *order = A.order + ((int64_t)row * A.chunks + c) * A.chunk_len;
-    for (int k = tid; k < cnt_c; k += kCT) order[k] = c0 + lorder[k];
+    uint16_t *order = A.order + ((int64_t)row * A.chunks + c) * A.chunk_len;
+    for (int k = tid; k < cnt_c; k += kCT) order[k] = lorder[k];
 }
 
 __global__ __launch_bounds__(kST) void sample_kernel(const SampleArgs A) {
@@ -416,6 +452,21 @@ __global__ __launch_bounds__(kST) void sample_kernel(const SampleArgs A) {
     const float *lg = row_logits(A, row);
     const int blocked = A.blocked ? A.blocked[row] : -1;
     const double T = A.temperature;
+    // The first chunks' histograms (thread t: buckets 2046-2t and 2047-2t), in
+    // flight while the history and the chunks' ranges are read.
+    constexpr int KB = 8;  // chunks' loads in flight
+    uint2 cc[KB];
+    ulonglong2 mm[KB];
+    auto load_hist = [&](int k0) {
+        const int64_t h = (int64_t)row * A.chunks * kBuckets + (kBuckets - 2 - 2 * tid);
+#pragma unroll
+        for (int k = 0; k < KB; ++k) {
+            const int64_t o = h + (int64_t)min(k0 + k, A.chunks - 1) * kBuckets;
+            cc[k] = *(const uint2 *)(A.hcount + o);
+            mm[k] = *(const ulonglong2 *)(A.hmass + o);
+        }
+    };
+    if (T != 0.0) load_hist(0);
     if (A.repeat_penalty != 1.0) seen_bits(A, row, 0, (vocab + 31) / 32, seen, kST);
     auto value = [&](int i, float x) { return penalised(A, seen, 0, i, x); };
 
@@ -459,7 +510,7 @@ __global__ __launch_bounds__(kST) void sample_kernel(const SampleArgs A) {
     if (bad || cnt == 0) {
         if (tid == 0) {
             A.ids[row] = -1;
-            atomicOr(A.err, bad ? 1 : 2);
+            A.err[row] = bad ? 1 : 2;
         }
         return;
     }
@@ -469,7 +520,28 @@ __global__ __launch_bounds__(kST) void sample_kernel(const SampleArgs A) {
     }
     // Integer mass of a candidate of value v: p = exp((v - vmax) / T) scaled
     // by 2^44 and rounded.
-    auto mass_of = [&](double v) { return (unsigned long long)(exp((v - vmax) / T) * kFix + 0.5); };
+    const MassOf mass_of(vmax, T);
+
+    // ---- the chunks' first-level histograms (pass B) ------------------------
+    // Thread t owns the buckets 2047-2t and 2046-2t over [vmin, vmax], in
+    // candidate order: their counts and masses, and the running totals before
+    // each.
+    unsigned long long hc[2] = {0, 0}, hm[2] = {0, 0}, hc_above[2], hm_above[2];
+    {
+        for (int k0 = 0;;) {
+#pragma unroll
+            for (int k = 0; k < KB; ++k)
+                if (k0 + k < A.chunks) {
+                    hc[0] += cc[k].y & 0xffffu, hc[1] += cc[k].x & 0xffffu;
+                    hm[0] += mm[k].y, hm[1] += mm[k].x;
+                }
+            if ((k0 += KB) >= A.chunks) break;
+            load_hist(k0);
+        }
+        hc_above[0] = block_scan(hc[0] + hc[1], s) - hc[0] - hc[1];
+        hm_above[0] = block_scan(hm[0] + hm[1], s) - hm[0] - hm[1];
+        hc_above[1] = hc_above[0] + hc[0], hm_above[1] = hm_above[0] + hm[0];
+    }
 
     // Candidates precede the bounds kcut (top_k) and pcut (top_p) in order.
     Cand kcut{-DBL_MAX, INT_MAX}, pcut{-DBL_MAX, INT_MAX};
@@ -479,12 +551,16 @@ __global__ __launch_bounds__(kST) void sample_kernel(const SampleArgs A) {
 
     // Locate the first candidate (in order) at which the running count or
     // mass satisfies the cut; s.cut / s.cum / s.found hold the result.
+    // CUT_COUNT: s.mcum is the mass of the candidates through the cut.
     auto locate = [&](int mode, unsigned long long target) {
         double lo = vmin, hi = vmax;
         double los[kLevels], scales[kLevels];
         int chosen[kLevels];
-        unsigned long long above = 0;
-        if (tid == 0) s.found = 0;
+        unsigned long long above = 0, mabove = 0;
+        auto hit = [&](unsigned long long c) { return mode == CUT_MASS_GT ? c > target : c >= target; };
+        __syncthreads();  // the last cut has been read
+        if (tid == 0) s.found = 0, s.bucket = INT_MAX;
+        __syncthreads();
         for (int level = 0; level < kLevels; ++level) {
             const double scale = hi > lo ? (double)kBuckets / (hi - lo) : 0.0;
             los[level] = lo;
@@ -495,8 +571,19 @@ __global__ __launch_bounds__(kST) void sample_kernel(const SampleArgs A) {
                 return true;
             };
             if (level == 0) {
-                // the first-level histogram of every candidate (pass B)
-                for (int b = tid; b < kBuckets; b += kST) s.hcount[b] = s.h0count[b], s.hmass[b] = s.h0mass[b];
+                // The first-level histogram (pass B): the running totals are
+                // in registers, and the one bucket in which the total
+                // reaches the target is its owner's to announce.
+#pragma unroll
+                for (int k = 1; k >= 0; --k) {
+                    const unsigned long long ex = mode == CUT_COUNT ? hc_above[k] : hm_above[k];
+                    if (hc[k] && hit(ex + (mode == CUT_COUNT ? hc[k] : hm[k])) && !hit(ex)) {
+                        s.bucket = 2 * tid + k;
+                        s.bucket_n = hc[k];
+                        s.above = ex;
+                        s.mabove = hm_above[k];
+                    }
+                }
                 __syncthreads();
             } else {
                 for (int b = tid; b < kBuckets; b += kST) s.hcount[b] = 0, s.hmass[b] = 0;
@@ -520,25 +607,25 @@ __global__ __launch_bounds__(kST) void sample_kernel(const SampleArgs A) {
                     }
                 }
                 __syncthreads();
-            }
-            // Running totals over buckets in descending order (bucket 2047
-            // first): thread t owns buckets 2047-2t and 2046-2t.
-            {
+                // Running totals over buckets in descending order (bucket 2047
+                // first): thread t owns buckets 2047-2t and 2046-2t.
                 const int b0 = kBuckets - 1 - 2 * tid, b1 = b0 - 1;
                 const unsigned long long w0 = mode == CUT_COUNT ? s.hcount[b0] : s.hmass[b0];
                 const unsigned long long w1 = mode == CUT_COUNT ? s.hcount[b1] : s.hmass[b1];
                 s.scan[tid] = block_scan(w0 + w1, s);  // inclusive
                 __syncthreads();
                 const unsigned long long before_t = above + (tid ? s.scan[tid - 1] : 0ull);
-                auto hit = [&](unsigned long long c) {
-                    return mode == CUT_MASS_GT ? c > target : c >= target;
-                };
                 // the first bucket (in order) whose inclusive total hits
                 int mine = INT_MAX;
                 if (hit(before_t + w0) && (w0 > 0 || mode == CUT_COUNT)) mine = 2 * tid;
                 else if (hit(before_t + w0 + w1)) mine = 2 * tid + 1;
                 if (mine != INT_MAX && s.hcount[kBuckets - 1 - mine] == 0) mine = INT_MAX;
                 const int first = block_min_int(mine, s);
+                // the mass of the buckets before it
+                unsigned long long mb = 0;
+                if (2 * tid < first) mb += s.hmass[b0];
+                if (2 * tid + 1 < first) mb += s.hmass[b1];
+                mb = block_sum(mb, s);
                 if (tid == 0) {
                     s.bucket = first;
                     if (first != INT_MAX) {
@@ -548,6 +635,8 @@ __global__ __launch_bounds__(kST) void sample_kernel(const SampleArgs A) {
                             a += mode == CUT_COUNT ? s.hcount[kBuckets - 1 - 2 * owner]
                                                    : s.hmass[kBuckets - 1 - 2 * owner];
                         s.above = a;
+                        s.mabove = mabove + mb;
+                        s.bucket_n = s.hcount[kBuckets - 1 - first];
                     }
                 }
                 __syncthreads();
@@ -555,8 +644,9 @@ __global__ __launch_bounds__(kST) void sample_kernel(const SampleArgs A) {
             if (s.bucket == INT_MAX) return;  // never reached: s.found stays 0
             const int b = kBuckets - 1 - s.bucket;
             above = s.above;
+            mabove = s.mabove;
             chosen[level] = b;
-            const uint32_t n = s.hcount[b];
+            const uint32_t n = s.bucket_n;
             if (n > (uint32_t)kList && level + 1 < kLevels && hi > lo) {
                 lo = lo + (double)b / scale;  // narrow to the bucket's value range
                 hi = lo + 1.0 / scale;
@@ -583,7 +673,7 @@ __global__ __launch_bounds__(kST) void sample_kernel(const SampleArgs A) {
                 __syncthreads();
                 const unsigned long long need = target - above;  // > 0: the cut lies in this bucket
                 if (bmn != bmx || (mode != CUT_COUNT && pe == 0)) {
-                    if (tid == 0) atomicOr(A.err, 4);
+                    if (tid == 0) A.err[row] = 4;
                     return;
                 }
                 const unsigned long long m = mode == CUT_COUNT    ? need
@@ -630,6 +720,7 @@ __global__ __launch_bounds__(kST) void sample_kernel(const SampleArgs A) {
                         if (rank == want) {
                             s.cut = Cand{bmn, id};
                             s.cum = above + (mode == CUT_COUNT ? m : m * pe);
+                            s.mcum = mabove + m * pe;
                             s.found = 1;
                         }
                     }
@@ -646,7 +737,7 @@ __global__ __launch_bounds__(kST) void sample_kernel(const SampleArgs A) {
                     uint32_t nk = 0, ok = 0;
                     if (tid < A.chunks) {
                         const int64_t hk = ((int64_t)row * A.chunks + tid) * kBuckets + b;
-                        nk = A.hcount[hk], ok = A.hoff[hk];
+                        nk = A.hcount[hk] & 0xffffu, ok = A.hcount[hk] >> 16;
                     }
                     uint32_t inc = nk;
 #pragma unroll
@@ -663,7 +754,8 @@ __global__ __launch_bounds__(kST) void sample_kernel(const SampleArgs A) {
                     int k = 0;  // the chunk whose share holds entry j
                     for (int w = kMaxChunks / 2; w > 0; w >>= 1)
                         if (k + w < A.chunks && s.cstart[k + w] <= j) k += w;
-                    const int i = A.order[((int64_t)row * A.chunks + k) * A.chunk_len + s.coff[k] + (j - s.cstart[k])];
+                    const int i = k * A.chunk_len +
+                                  A.order[((int64_t)row * A.chunks + k) * A.chunk_len + s.coff[k] + (j - s.cstart[k])];
                     const double v = value(i, lg[i]);
                     if (!member(i, v)) continue;
                     const int q = atomicAdd(&s.list_n, 1);
@@ -690,31 +782,37 @@ __global__ __launch_bounds__(kST) void sample_kernel(const SampleArgs A) {
             }
             __syncthreads();
             const int ln = s.list_n;
-            int pw = 1;
-            while (pw < ln) pw <<= 1;
             if (ln <= kRankSort) {
-                // Few candidates: each one's rank (the candidates before it,
-                // counted by 8 threads over every 8th entry), then each is
-                // stored at its rank.
+                // Few candidates: each one's running totals directly, the
+                // counts and masses of the candidates before it summed by 8
+                // threads over every 8th entry.  One candidate's total
+                // reaches the target.
                 const int e = tid >> 3, q = tid & 7;
                 double ev = 0.0;
-                int eid = 0, rank = 0;
-                unsigned long long ep = 0;
+                int eid = 0;
+                unsigned long long ep = 0, cb = 0, mb = 0;
                 if (e < ln) {
                     ev = s.lv[e], eid = s.li[e], ep = s.lp[e];
-                    for (int j = q; j < ln; j += 8) rank += before(s.lv[j], s.li[j], ev, eid);
+                    for (int j = q; j < ln; j += 8)
+                        if (before(s.lv[j], s.li[j], ev, eid)) ++cb, mb += s.lp[j];
                 }
-                rank += __shfl_xor(rank, 1, 64);
-                rank += __shfl_xor(rank, 2, 64);
-                rank += __shfl_xor(rank, 4, 64);
+#pragma unroll
+                for (int o = 1; o < 8; o <<= 1) cb += __shfl_xor(cb, o, 64), mb += __shfl_xor(mb, o, 64);
+                const unsigned long long ex = above + (mode == CUT_COUNT ? cb : mb);
+                const unsigned long long in = ex + (mode == CUT_COUNT ? 1ull : ep);
+                if (e < ln && q == 0 && hit(in) && !hit(ex)) {
+                    s.cut = Cand{ev, eid};
+                    s.cum = in;
+                    s.mcum = mabove + mb + ep;
+                    s.found = 1;
+                }
                 __syncthreads();
-                if (e < ln && q == 0) s.lv[rank] = ev, s.li[rank] = eid, s.lp[rank] = ep;
-                __syncthreads();
-                pw = 1;  // sorted
-            } else {
-                for (int k = ln + tid; k < pw; k += kST) s.lv[k] = -DBL_MAX, s.li[k] = INT_MAX, s.lp[k] = 0;
-                __syncthreads();
+                return;
             }
+            int pw = 1;
+            while (pw < ln) pw <<= 1;
+            for (int k = ln + tid; k < pw; k += kST) s.lv[k] = -DBL_MAX, s.li[k] = INT_MAX, s.lp[k] = 0;
+            __syncthreads();
             for (int size = 2; size <= pw; size <<= 1) {  // bitonic sort into candidate order
                 for (int stride = size >> 1; stride > 0; stride >>= 1) {
                     for (int k = tid; k < pw; k += kST) {
@@ -744,7 +842,6 @@ __global__ __launch_bounds__(kST) void sample_kernel(const SampleArgs A) {
                 s.scan[tid] = block_scan(w0 + w1, s);  // inclusive
                 __syncthreads();
                 const unsigned long long c0 = above + (tid ? s.scan[tid - 1] : 0ull) + w0, c1 = c0 + w1;
-                auto hit = [&](unsigned long long c) { return mode == CUT_MASS_GT ? c > target : c >= target; };
                 const int mine = k0 < ln && hit(c0) ? k0 : k1 < ln && hit(c1) ? k1 : INT_MAX;
                 const int first = block_min_int(mine, s);
                 if (first != INT_MAX && mine == first) {
@@ -752,52 +849,26 @@ __global__ __launch_bounds__(kST) void sample_kernel(const SampleArgs A) {
                     s.cum = (first & 1) ? c1 : c0;
                     s.found = 1;
                 }
+                if (mode == CUT_COUNT) {
+                    const unsigned long long mb = block_sum((k0 <= first && k0 < ln ? s.lp[k0] : 0ull) +
+                                                                (k1 <= first && k1 < ln ? s.lp[k1] : 0ull), s);
+                    if (tid == 0) s.mcum = mabove + mb;
+                }
             }
             __syncthreads();
             return;
         }
     };
 
-    // ---- the chunks' total mass and first-level histograms (pass B) ---------
-    // (buckets over [vmin, vmax], as locate's first level computes them)
-    {
-        uint32_t c0 = 0, c1 = 0;
-        unsigned long long m0 = 0, m1 = 0;
-        const int64_t h = (int64_t)row * A.chunks * kBuckets + 2 * tid;
-        constexpr int KB = 16;  // chunks' loads in flight
-        for (int k0 = 0; k0 < A.chunks; k0 += KB) {
-            uint2 cc[KB];
-            ulonglong2 mm[KB];
-#pragma unroll
-            for (int k = 0; k < KB; ++k) {
-                const int64_t o = h + (int64_t)min(k0 + k, A.chunks - 1) * kBuckets;
-                cc[k] = *(const uint2 *)(A.hcount + o);
-                mm[k] = *(const ulonglong2 *)(A.hmass + o);
-            }
-#pragma unroll
-            for (int k = 0; k < KB; ++k)
-                if (k0 + k < A.chunks) c0 += cc[k].x, c1 += cc[k].y, m0 += mm[k].x, m1 += mm[k].y;
-        }
-        s.h0count[2 * tid] = c0, s.h0count[2 * tid + 1] = c1;
-        s.h0mass[2 * tid] = m0, s.h0mass[2 * tid + 1] = m1;
-    }
-    __syncthreads();  // the cuts read every thread's buckets
-
     // top_k: keep the first k candidates (M:7390-7395).
     if (A.top_k > 0 && A.top_k < cnt) {
         locate(CUT_COUNT, (unsigned long long)A.top_k);
         if (!s.found) {
-            if (tid == 0) atomicOr(A.err, 8), A.ids[row] = -1;
+            if (tid == 0) A.err[row] = 8, A.ids[row] = -1;
             return;
         }
         kcut = s.cut;
-        // mass of the kept candidates
-        unsigned long long m = 0;
-        for (int i = tid; i < vocab; i += kST) {
-            const double v = value(i, lg[i]);
-            if (member(i, v)) m += mass_of(v);
-        }
-        total = block_sum(m, s);
+        total = s.mcum;  // mass of the kept candidates
     }
     // top_p: the shortest prefix with mass >= top_p * total (M:7398-7409).
     if (A.top_p < 1.0) {
@@ -832,15 +903,15 @@ __global__ __launch_bounds__(kST) void sample_kernel(const SampleArgs A) {
     }
     if (tid == 0) {
         A.ids[row] = id;
-        A.rng[row] = st;
+        A.rng_out[row] = st;
     }
 }
 
 }  // namespace
 
 void sample_plan(int32_t rows, int32_t vocab, int32_t &chunks, int32_t &chunk_len) {
-    // About 512 chunk workgroups, chunks of at least 2048 ids.
-    int c = (int)std::min<int64_t>(kMaxChunks, std::max<int64_t>(1, (512 + rows - 1) / rows));
+    // About 256 chunk workgroups (one per CU), chunks of at least 2048 ids.
+    int c = (int)std::min<int64_t>(kMaxChunks, std::max<int64_t>(1, (256 + rows - 1) / rows));
     c = (int)std::min<int64_t>(c, (vocab + 2047) / 2048);
     c = (int)std::max<int64_t>({(int64_t)c, 1, ((int64_t)vocab + kChunkMax - 1) / kChunkMax});
     chunk_len = (vocab + c - 1) / c;
@@ -852,8 +923,8 @@ static size_t plan_bytes(int32_t rows, int32_t vocab) {
     int32_t chunks, len;
     sample_plan(rows, vocab, chunks, len);
     return (size_t)rows * chunks *
-           (sizeof(SampleRange) + kBuckets * (sizeof(unsigned long long) + 2 * sizeof(uint32_t)) +
-            (size_t)len * sizeof(int32_t));
+           (sizeof(SampleRange) + kBuckets * (sizeof(unsigned long long) + sizeof(uint32_t)) +
+            (size_t)len * sizeof(uint16_t));
 }
 
 // Rows per launch group: the most (a power of two up to 1024) whose scratch
@@ -889,18 +960,19 @@ int launch_sample(hipStream_t s, const SampleArgs &a0, void *scratch) {
         if (a0.history_len) a.history_len = a0.history_len + r0;
         if (a0.blocked) a.blocked = a0.blocked + r0;
         a.rng = a0.rng + r0;
+        a.rng_out = a0.rng_out + r0;
         a.ids = a0.ids + r0;
+        a.err = a0.err + r0;
         sample_plan(a.rows, a.vocab, a.chunks, a.chunk_len);
         if (a.chunks > kMaxChunks || a.chunk_len > kChunkMax)
             return fail(SRQ_EINVAL, "sample: vocabulary of %d ids exceeds the chunk plan", a.vocab);
-        // [ranges: rows x chunks][masses: rows x chunks x 2048][counts: likewise]
-        // [offsets: likewise][ids in bucket order: rows x chunks x chunk_len]
+        // [ranges: rows x chunks][masses: rows x chunks x 2048][counts and
+        // offsets: likewise][ids in bucket order: rows x chunks x chunk_len]
         const size_t nb = (size_t)a.rows * a.chunks * kBuckets;
         a.range = (SampleRange *)scratch;
         a.hmass = (unsigned long long *)(a.range + (size_t)a.rows * a.chunks);
         a.hcount = (uint32_t *)(a.hmass + nb);
-        a.hoff = a.hcount + nb;
-        a.order = (int32_t *)(a.hoff + nb);
+        a.order = (uint16_t *)(a.hcount + nb);
         const size_t clds = (size_t)((a.chunk_len + 31) / 32) * 4;
         const dim3 grid(a.chunks, a.rows);
         sample_range_kernel<<<grid, kCT, a.repeat_penalty != 1.0 ? clds : 0, s>>>(a);

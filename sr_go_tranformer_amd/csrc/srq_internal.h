@@ -218,17 +218,19 @@ struct SampleArgs {
     const int32_t *history_len;  // [rows] or null
     int32_t history_stride;
     const int32_t *blocked;      // [rows] (-1: none) or null
-    uint64_t *rng;               // [rows] SplitMix64 states, advanced per draw
-    int32_t *ids;                // [rows] out
-    int32_t *err;                // |= 1 non-finite logit, 2 no candidate, 4/8 selection limits
+    const uint64_t *rng;         // [rows] SplitMix64 states
+    // Results, in pinned host memory: each row's one thread writes them, and
+    // no copy follows the kernels.
+    uint64_t *rng_out;           // [rows] the states advanced, written where a row draws
+    int32_t *ids;                // [rows]
+    int32_t *err;                // [rows] 1 non-finite logit, 2 no candidate, 4/8 selection limits, else unwritten
     // Set by launch_sample: rows are cut into `chunks` chunks of chunk_len
     // ids, each chunk's range and histogram kept in scratch.
     int32_t chunks, chunk_len;
     struct SampleRange *range;   // [rows x chunks]
     unsigned long long *hmass;   // [rows x chunks x 2048]
-    uint32_t *hcount;            // [rows x chunks x 2048]
-    uint32_t *hoff;              // [rows x chunks x 2048] bucket starts in `order`
-    int32_t *order;              // [rows x chunks x chunk_len] a chunk's candidate ids by bucket
+    uint32_t *hcount;            // [rows x chunks x 2048] count | start in `order` << 16
+    uint16_t *order;             // [rows x chunks x chunk_len] a chunk's candidates (less its first id) by bucket
 };
 struct SampleRange {  // one chunk of a row
     double vmax, vmin, best_v;

@@ -191,3 +191,24 @@ def test_sample_flat_rows_rank_by_id(ex):
         want, wst = oracle_rows(logits, t, k, p, 1.0, seeds)
         assert np.array_equal(got, want), (t, k, p, got, want)
         assert np.array_equal(gst, wst)
+
+
+@pytest.mark.parametrize("vocab", [2049, 16385, 40000])
+@pytest.mark.parametrize("spread", [0.0, 1e-3, 3.0])
+def test_sample_crowded_buckets(ex, vocab, spread):
+    """One far low value stretches the range, so that the other ids share a few
+    first-level buckets (spread 0: one): top_k's mass comes from refined
+    levels, from a sort of up to 2048 candidates or from a run of equal
+    values; chunks of one id to a full one."""
+    rng = np.random.default_rng(vocab)
+    rows = 4
+    logits = rng.normal(0, spread, size=(rows, vocab)).astype(np.float32)
+    logits[:2, 17] = -500.0
+    seeds = rng.integers(0, 2**63, size=rows, dtype=np.uint64)
+    hist = [list(rng.integers(0, vocab, size=9)) for _ in range(rows)]
+    for t, k, p, rp in [(0.8, 40, 0.95, 1.1), (1.0, 1500, 0.5, 1.0), (0.9, 0, 0.7, 1.2), (0.3, vocab - 1, 0.99, 1.0)]:
+        print("crowded", vocab, spread, t, k, p, rp, flush=True)
+        got, gst = run(ex, logits, srq.Sampling(t, k, p, rp), seeds, hist)
+        want, wst = oracle_rows(logits, t, k, p, rp, seeds, hist)
+        assert np.array_equal(got, want), (t, k, p, got, want)
+        assert np.array_equal(gst, wst)

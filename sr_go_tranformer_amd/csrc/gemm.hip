@@ -1,15 +1,17 @@
-// Dequant-GEMM on FP32 MFMA for prefill chunks and batched steps (n > 16).
+// Dequant-GEMM on MFMA for prefill chunks and batched steps (n > 16), and the
+// plan and reductions that the tall tiles (gemm_tall.hip) and F32 weights
+// (gemm_f32.hip) share.
 //
-// Counterpart of linearQ8Into / linearQ4Into / linearFP32Range
-// (cmd/monolith/monolith.go M:3942-4780) when many activation rows share
-// each weight read.
+// Counterpart of linearQ8Into / linearQ4Into (cmd/monolith/monolith.go
+// M:3942-4780) when many activation rows share each weight read.
 //
-// Tiling (gfx950, wave64, v_mfma_f32_16x16x4f32):
+// Tiling of gemm_kernel, for Q8 / Q4 widths that are no multiple of 64 (gfx950,
+// wave64, v_mfma_f32_16x16x4f32):
 //  - Workgroup tile BMT (activation rows: 32 when n <= 32, else 64) x 128
 //    (output features), K step 32 (half a scale block).  4 waves; each owns
 //    32 rows x (128 / waves across N) features as 16x16 MFMA tiles with FP32
 //    accumulators.
-//  - Weights are read once per K step as int8 / packed int4 / f32,
+//  - Weights are read once per K step as int8 / packed int4,
 //    dequantised in registers to f32(code)*scale (the copyRow rounding,
 //    M:3900-3921) and stored to LDS; activations go to LDS unchanged.
 //  - Within a K step, MFMA step s feeds lane group g (lane/16) the K index
@@ -39,43 +41,38 @@ constexpr int kMinSliceInputs = 256;  // inputs per split-K slice, at least
 
 template <int FMT>
 __device__ __forceinline__ void load_b(const uint8_t *__restrict__ W, const float *__restrict__ S, int64_t rows,
-                                       int64_t cols, int64_t n0, int64_t k0, int tid, uint4 (&raw)[4],
+                                       int64_t cols, int64_t n0, int64_t k0, int tid, uint4 &raw,
                                        float &scale) {
     const int r = tid >> 1, half = tid & 1;
     const int64_t row = n0 + r;
     if (row >= rows) {
-        raw[0] = raw[1] = raw[2] = raw[3] = make_uint4(0, 0, 0, 0);
+        raw = make_uint4(0, 0, 0, 0);
         scale = 0.0f;
         return;
     }
     if constexpr (FMT == SRQ_Q8) {
-        raw[0] = ld_stream16(W + row * cols + k0 + 16 * half);
-        scale = S[row * groups_of(cols) + k0 / kBlock];
-    } else if constexpr (FMT == SRQ_Q4) {
-        const uint2 v = ld_stream8(W + row * (cols / 2) + k0 / 2 + 8 * half);
-        raw[0] = make_uint4(v.x, v.y, 0, 0);
+        raw = ld_stream16(W + row * cols + k0 + 16 * half);
         scale = S[row * groups_of(cols) + k0 / kBlock];
     } else {
-        const uint4 *p = (const uint4 *)(W + (row * cols + k0 + 16 * half) * 4);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) raw[i] = ld_stream16(p + i);
-        scale = 1.0f;
+        const uint2 v = ld_stream8(W + row * (cols / 2) + k0 / 2 + 8 * half);
+        raw = make_uint4(v.x, v.y, 0, 0);
+        scale = S[row * groups_of(cols) + k0 / kBlock];
     }
 }
 
 template <int FMT>
-__device__ __forceinline__ void store_b(float *Bs, int tid, const uint4 (&raw)[4], float scale) {
+__device__ __forceinline__ void store_b(float *Bs, int tid, const uint4 &raw, float scale) {
     const int r = tid >> 1, half = tid & 1;
     float *dst = Bs + r * LDK + 16 * half;
     float w[16];
     if constexpr (FMT == SRQ_Q8) {
-        const uint32_t d[4] = {raw[0].x, raw[0].y, raw[0].z, raw[0].w};
+        const uint32_t d[4] = {raw.x, raw.y, raw.z, raw.w};
 #pragma unroll
         for (int k = 0; k < 4; ++k)
 #pragma unroll
             for (int b = 0; b < 4; ++b) w[4 * k + b] = (float)(int32_t)(int8_t)(d[k] >> (8 * b)) * scale;
-    } else if constexpr (FMT == SRQ_Q4) {
-        const uint32_t d[2] = {raw[0].x, raw[0].y};
+    } else {
+        const uint32_t d[2] = {raw.x, raw.y};
 #pragma unroll
         for (int k = 0; k < 2; ++k)
 #pragma unroll
@@ -84,14 +81,6 @@ __device__ __forceinline__ void store_b(float *Bs, int tid, const uint4 (&raw)[4
                 w[8 * k + 2 * b] = (float)(((int32_t)(byte << 28)) >> 28) * scale;
                 w[8 * k + 2 * b + 1] = (float)(((int32_t)(byte << 24)) >> 28) * scale;
             }
-    } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            w[4 * i + 0] = __uint_as_float(raw[i].x);
-            w[4 * i + 1] = __uint_as_float(raw[i].y);
-            w[4 * i + 2] = __uint_as_float(raw[i].z);
-            w[4 * i + 3] = __uint_as_float(raw[i].w);
-        }
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) *(float4 *)(dst + 4 * i) = make_float4(w[4 * i], w[4 * i + 1], w[4 * i + 2], w[4 * i + 3]);
@@ -161,7 +150,7 @@ __global__ __launch_bounds__(256) void gemm_kernel(const GemmArgs G, float *__re
 #pragma unroll
         for (int j = 0; j < TN; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
 
-    uint4 braw[4];
+    uint4 braw;
     float bscale;
     float4 areg[NV];
     load_b<FMT>(W, G.scales, G.rows, cols, n0, (int64_t)kbeg * BK, tid, braw, bscale);
@@ -209,46 +198,7 @@ __global__ __launch_bounds__(256) void gemm_kernel(const GemmArgs G, float *__re
     if (amax > kWideLimit) row_wide[tid / ATile<BMT>::TPR] = 1;
     __syncthreads();
 
-    // D layout of 16x16x4: lane holds rows 4*(lane/16)+r, column lane%16.
-    if (partial) {
-        float *P = partial + (int64_t)blockIdx.z * G.n * G.rows;
-        if (blockIdx.x == 0 && tid < BMT && m0 + tid < G.n) wflags[(int64_t)blockIdx.z * G.n + m0 + tid] = row_wide[tid];
-#pragma unroll
-        for (int tm = 0; tm < 2; ++tm)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int64_t m = m0 + wm * 32 + tm * 16 + 4 * gq + r;
-                if (m >= G.n) continue;
-#pragma unroll
-                for (int tn = 0; tn < TN; ++tn) {
-                    const int64_t j = n0 + wn * TN * 16 + tn * 16 + li;
-                    if (j < G.rows) P[m * G.rows + j] = acc[tm][tn][r];
-                }
-            }
-        return;
-    }
-#pragma unroll
-    for (int tm = 0; tm < 2; ++tm)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int mi = wm * 32 + tm * 16 + 4 * gq + r;
-            const int64_t m = m0 + mi;
-            if (m >= G.n || row_wide[mi]) continue;
-#pragma unroll
-            for (int tn = 0; tn < TN; ++tn) {
-                const int64_t j = n0 + wn * TN * 16 + tn * 16 + li;
-                if (j >= G.rows) continue;
-                float v = acc[tm][tn][r];
-                if (G.residual) v = G.residual[m * G.y_stride + j] + v;
-                G.y[m * G.y_stride + j] = v;
-            }
-        }
-    // This workgroup saw all of K: it recomputes its wide rows itself.
-    for (int mi = 0; mi < BMT; ++mi) {
-        if (!row_wide[mi] || m0 + mi >= G.n) continue;
-        const int64_t j = n0 + tid;
-        if (tid < BN && j < G.rows) G.y[(m0 + mi) * G.y_stride + j] = wide_output(G, m0 + mi, j);
-    }
+    gemm_finish<BMT, BN, 2, TN>(G, partial, wflags, acc, row_wide, n0, m0, wm * 32, wn * TN * 16, tid);
 }
 
 // Sum over the K slices z of p[z * plane], added in slice order.  The loads
@@ -1128,11 +1078,7 @@ void launch_pairs(hipStream_t s, dim3 grid, const GemmArgs &a, float *partial, i
 
 template <int FMT, int BMT>
 void launch_tiles(hipStream_t s, const GemmArgs &a, const GemmPlan &p, float *partial, int32_t *wflags) {
-    static_assert(BMT >= 32 || FMT != SRQ_F32, "16-row tiles are the bf16 kernel's");
-    if constexpr (FMT == SRQ_F32) {
-        dim3 grid((unsigned)((a.rows + BN - 1) / BN), (unsigned)((a.n + BMT - 1) / BMT), (unsigned)p.slices);
-        gemm_kernel<FMT, BMT><<<grid, 256, 0, s>>>(a, partial, wflags, p.kper);
-    } else {
+    {
         if (p.x3) {
             const int xbn = 64 * p.tn;
             dim3 grid((unsigned)((a.rows + xbn - 1) / xbn), (unsigned)((a.n + BMT - 1) / BMT), (unsigned)p.slices);
@@ -1209,9 +1155,7 @@ void launch_fmt(hipStream_t s, const GemmArgs &a, const GemmPlan &p, float *part
     switch (a.fmt) {
         case SRQ_Q8: launch_tiles<SRQ_Q8, BMT>(s, a, p, partial, wflags); break;
         case SRQ_Q4: launch_tiles<SRQ_Q4, BMT>(s, a, p, partial, wflags); break;
-        default:
-            if constexpr (BMT >= 32) launch_tiles<SRQ_F32, BMT>(s, a, p, partial, wflags);
-            break;
+        default: break;  // F32: launch_gemm_f32
     }
 }
 
@@ -1286,6 +1230,8 @@ int launch_gemm(hipStream_t s, const GemmArgs &a, void *scratch, size_t scratch_
         if (!wflags) wflags = (int32_t *)scratch;
         SRQ_CHECK(launch_gemm_tall(s, a, tall_plan(a.n, a.rows, p.slices), (uint8_t *)scratch + off, partial, wflags,
                                    p.slices, p.kper));
+    } else if (a.fmt == SRQ_F32) {
+        SRQ_CHECK(launch_gemm_f32(s, a, partial, wflags, p.slices, p.kper));
     } else if (p.bm == 16) {
         launch_fmt<16>(s, a, p, partial, wflags);  // bf16 kernel only (plan_gemm)
     } else if (p.bm == 32) {

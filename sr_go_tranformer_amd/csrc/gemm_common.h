@@ -1,4 +1,4 @@
-// Device code shared by the GEMM kernels (gemm.hip, gemm_tall.hip).
+// Device code shared by the GEMM kernels (gemm.hip, gemm_tall.hip, gemm_f32.hip).
 #pragma once
 
 #include "srq_internal.h"
@@ -38,6 +38,58 @@ __device__ __forceinline__ float wide_output(const GemmArgs &G, int64_t m, int64
     return v;
 }
 
+// Stores a workgroup's MFMA tiles: partial sums of its K slice (partial !=
+// nullptr; wide-row flags from the first feature tile), else y (+ residual),
+// rows holding a |x| > kWideLimit recomputed in FP64.  D layout of the 16x16
+// MFMAs: lane holds rows 4*(lane/16)+r, column lane%16.  BM rows x BN features
+// from (m0, n0); this wave's TM x TN tiles start at (mw, nw) of them.
+template <int BM, int BN, int TM, int TN>
+__device__ __forceinline__ void gemm_finish(const GemmArgs &G, float *__restrict__ partial,
+                                            int32_t *__restrict__ wflags, const floatx4 (&acc)[TM][TN],
+                                            const int *row_wide, const int64_t n0, const int64_t m0, const int mw,
+                                            const int nw, const int tid) {
+    const int li = tid & 15, gq = (tid & 63) >> 4;
+    if (partial) {
+        float *P = partial + (int64_t)blockIdx.z * G.n * G.rows;
+        if (blockIdx.x == 0 && tid < BM && m0 + tid < G.n) wflags[(int64_t)blockIdx.z * G.n + m0 + tid] = row_wide[tid];
+#pragma unroll
+        for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int64_t m = m0 + mw + tm * 16 + 4 * gq + r;
+                if (m >= G.n) continue;
+#pragma unroll
+                for (int tn = 0; tn < TN; ++tn) {
+                    const int64_t j = n0 + nw + tn * 16 + li;
+                    if (j < G.rows) P[m * G.rows + j] = acc[tm][tn][r];
+                }
+            }
+        return;
+    }
+#pragma unroll
+    for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int mi = mw + tm * 16 + 4 * gq + r;
+            const int64_t m = m0 + mi;
+            if (m >= G.n || row_wide[mi]) continue;
+#pragma unroll
+            for (int tn = 0; tn < TN; ++tn) {
+                const int64_t j = n0 + nw + tn * 16 + li;
+                if (j >= G.rows) continue;
+                float v = acc[tm][tn][r];
+                if (G.residual) v = G.residual[m * G.y_stride + j] + v;
+                G.y[m * G.y_stride + j] = v;
+            }
+        }
+    // This workgroup saw all of K: it recomputes its wide rows itself.
+    for (int mi = 0; mi < BM; ++mi) {
+        if (!row_wide[mi] || m0 + mi >= G.n) continue;
+        const int64_t j = n0 + tid;
+        if (tid < BN && j < G.rows) G.y[(m0 + mi) * G.y_stride + j] = wide_output(G, m0 + mi, j);
+    }
+}
+
 // Workgroup barrier over LDS only.  __syncthreads() also waits for every
 // global load in flight (vmcnt(0)), which in the block loop below would
 // drain the weight and activation loads issued blocks ahead at every block.
@@ -45,6 +97,26 @@ __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// LDS-direct loads: 16 (4) bytes per lane from base + voff (32-bit, per lane)
+// to lds + 16 (4) * lane.  In asm because the compiler would make every later
+// LDS read wait for them; the block loop waits for them itself.
+__device__ __forceinline__ void lds_load16(uint32_t lds, uint32_t voff, const uint8_t *base) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                 :
+                 : "s"(lds), "v"(voff), "s"(base)
+                 : "memory");
+}
+__device__ __forceinline__ void lds_load4(uint32_t lds, uint32_t voff, const uint8_t *base) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
+                 :
+                 : "s"(lds), "v"(voff), "s"(base)
+                 : "memory");
+}
+// The same 16 bytes from an address per lane.
+__device__ __forceinline__ void lds_load16(uint32_t lds, const uint8_t *p) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(lds), "v"(p) : "memory");
 }
 
 __device__ __forceinline__ uint32_t pk_hi16(float lo, float hi) {
@@ -108,5 +180,8 @@ size_t tall_plane_bytes(const TallPlan &p, int32_t n, int64_t cols);
 // wflags: slices * n words; partial as gemm_x3_kernel's (null: writes y).
 int launch_gemm_tall(hipStream_t s, const GemmArgs &a, const TallPlan &p, uint8_t *planes, float *partial,
                      int32_t *wflags, int slices, int kper);
+
+// gemm_f32.hip: F32 weights, cols % 32 == 0; kper counts K steps of 32.
+int launch_gemm_f32(hipStream_t s, const GemmArgs &a, float *partial, int32_t *wflags, int slices, int kper);
 
 }  // namespace srq

@@ -71,21 +71,6 @@ __global__ __launch_bounds__(kSplitThreads) void gemm_split_kernel(const float *
     for (int z = threadIdx.x; z < slices; z += kSplitThreads) wflags[(int64_t)z * n + m] = wide;
 }
 
-// LDS-direct loads: 16 (4) bytes per lane from base + voff (32-bit, per lane)
-// to lds + 16 (4) * lane.  In asm because the compiler would make every later
-// LDS read wait for them; the block loop waits for them itself.
-__device__ __forceinline__ void lds_load16(uint32_t lds, uint32_t voff, const uint8_t *base) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                 :
-                 : "s"(lds), "v"(voff), "s"(base)
-                 : "memory");
-}
-__device__ __forceinline__ void lds_load4(uint32_t lds, uint32_t voff, const uint8_t *base) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
-                 :
-                 : "s"(lds), "v"(voff), "s"(base)
-                 : "memory");
-}
 // lds_load16 unless `skip` (uniform) is not 0.  The branch is inside the asm:
 // around it, the compiler would keep two copies of the accumulators.
 __device__ __forceinline__ void lds_load16_unless(uint32_t skip, uint32_t lds, uint32_t voff, const uint8_t *base) {

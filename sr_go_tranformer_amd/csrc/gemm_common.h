@@ -181,6 +181,12 @@ size_t tall_plane_bytes(const TallPlan &p, int32_t n, int64_t cols);
 int launch_gemm_tall(hipStream_t s, const GemmArgs &a, const TallPlan &p, uint8_t *planes, float *partial,
                      int32_t *wflags, int slices, int kper);
 
+// gemm_pairs.hip: calls of at most 32 rows (bm 16 or 32, tn as plan_gemm's)
+// whose weights it can read by 128-byte row segments.
+bool gemm_pairs_ok(const GemmArgs &a, int kper);
+void launch_gemm_pairs(hipStream_t s, const GemmArgs &a, int bm, int tn, float *partial, int32_t *wflags, int slices,
+                       int kper);
+
 // gemm_f32.hip: F32 weights, cols % 32 == 0; kper counts K steps of 32.
 int launch_gemm_f32(hipStream_t s, const GemmArgs &a, float *partial, int32_t *wflags, int slices, int kper);
 

@@ -741,29 +741,18 @@ __device__ __forceinline__ int stage_stream(const GemvArgs &A, float *lds, const
     return mask & ((1 << A.n) - 1);
 }
 
-// Write one unit's results: lane b (b < NB, b < n, write) stores batch
-// row b; values v[i][b] are wave-uniform.  resid: lane b's residual values
-// of the unit's rows (EPI_RESID).  No global loads: operands come from LDS
-// or the load stream.
-template <int EPI, int NB, int R>
-__device__ __forceinline__ void unit_epilogue(const GemvArgs &A, const Unit &t, const float (&v)[R][NB],
-                                              const float *lds, const StreamLds &L, const StreamSmem &sm,
-                                              float resid, int lane, bool write) {
-    if (!(write && lane < NB && lane < A.n)) return;
+// Operands of one batch row's epilogue (EPI_ROPE_KV): its position's {cos, sin}
+// of the unit's pair, the rows' bias and the row's KV offset.
+struct EpiOps {
+    float c, s, bias0, bias1;
+    int64_t kvoff;
+};
+
+// Write one unit's results vv of a batch row whose output row is yb.
+template <int EPI, int R>
+__device__ __forceinline__ void store_unit(const GemvArgs &A, const Unit &t, float *yb, const float (&vv)[R],
+                                           float resid, const EpiOps &o) {
     const int *r = t.r;
-    const int b = lane;
-    // vv[i] = v[i][b]: an OR of masked bit patterns (exactly one term is
-    // nonzero), which stays in registers (an indexed pick would go through
-    // scratch memory).
-    float vv[R];
-#pragma unroll
-    for (int i = 0; i < R; ++i) {
-        uint32_t bits = 0;
-#pragma unroll
-        for (int bb = 0; bb < NB; ++bb) bits |= b == bb ? __float_as_uint(v[i][bb]) : 0u;
-        vv[i] = __uint_as_float(bits);
-    }
-    float *yb = A.y + (int64_t)b * A.y_stride;
     if constexpr (EPI == EPI_PLAIN) {
         yb[r[0]] = vv[0];
     } else if constexpr (EPI == EPI_RESID) {
@@ -776,15 +765,13 @@ __device__ __forceinline__ void unit_epilogue(const GemvArgs &A, const Unit &t, 
     } else {  // EPI_ROPE_KV
         float a = vv[0], z = vv[R - 1];
         if (A.bias) {
-            a = __fadd_rn(a, lds[L.bias + r[0]]);
-            z = __fadd_rn(z, lds[L.bias + r[1]]);
+            a = __fadd_rn(a, o.bias0);
+            z = __fadd_rn(z, o.bias1);
         }
         if (t.j >= 0) {
-            const float c = lds[L.rope + b * A.head_dim + 2 * t.j];
-            const float sn = lds[L.rope + b * A.head_dim + 2 * t.j + 1];
             // x' = a*c - z*s ; z' = a*s + z*c  (M:5283-5285), unfused
-            const float na = __fsub_rn(__fmul_rn(a, c), __fmul_rn(z, sn));
-            const float nz = __fadd_rn(__fmul_rn(a, sn), __fmul_rn(z, c));
+            const float na = __fsub_rn(__fmul_rn(a, o.c), __fmul_rn(z, o.s));
+            const float nz = __fadd_rn(__fmul_rn(a, o.s), __fmul_rn(z, o.c));
             a = na;
             z = nz;
         }
@@ -793,7 +780,7 @@ __device__ __forceinline__ void unit_epilogue(const GemvArgs &A, const Unit &t, 
             yb[r[0]] = a;
             yb[r[1]] = z;
         } else {
-            float *kv = A.meta.kv_pool + sm.kvoff[b] + (int64_t)A.meta.layer * 2 * kPageTokens * A.kvdim;
+            float *kv = A.meta.kv_pool + o.kvoff + (int64_t)A.meta.layer * 2 * kPageTokens * A.kvdim;
             if (r[0] < qk_rows) {
                 kv[r[0] - A.dim] = a;
                 kv[r[1] - A.dim] = z;
@@ -804,6 +791,39 @@ __device__ __forceinline__ void unit_epilogue(const GemvArgs &A, const Unit &t, 
             }
         }
     }
+}
+
+// Write one unit's results: lane b (b < NB, b < n, write) stores batch
+// row b; values v[i][b] are wave-uniform.  resid: lane b's residual values
+// of the unit's rows (EPI_RESID).  No global loads: operands come from LDS
+// or the load stream.
+template <int EPI, int NB, int R>
+__device__ __forceinline__ void unit_epilogue(const GemvArgs &A, const Unit &t, const float (&v)[R][NB],
+                                              const float *lds, const StreamLds &L, const StreamSmem &sm,
+                                              float resid, int lane, bool write) {
+    if (!(write && lane < NB && lane < A.n)) return;
+    const int b = lane;
+    // vv[i] = v[i][b]: an OR of masked bit patterns (exactly one term is
+    // nonzero), which stays in registers (an indexed pick would go through
+    // scratch memory).
+    float vv[R];
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+        uint32_t bits = 0;
+#pragma unroll
+        for (int bb = 0; bb < NB; ++bb) bits |= b == bb ? __float_as_uint(v[i][bb]) : 0u;
+        vv[i] = __uint_as_float(bits);
+    }
+    EpiOps o = {};
+    if constexpr (EPI == EPI_ROPE_KV) {
+        if (A.bias) o.bias0 = lds[L.bias + t.r[0]], o.bias1 = lds[L.bias + t.r[1]];
+        if (t.j >= 0) {
+            o.c = lds[L.rope + b * A.head_dim + 2 * t.j];
+            o.s = lds[L.rope + b * A.head_dim + 2 * t.j + 1];
+        }
+        o.kvoff = sm.kvoff[b];
+    }
+    store_unit<EPI, R>(A, t, A.y + (int64_t)b * A.y_stride, vv, resid, o);
 }
 
 // G: chunks that share one load of block scales.  A step's lane needs the
@@ -1097,6 +1117,246 @@ __global__ __launch_bounds__(kStreamThreads) void gemv_stream_kernel(const GemvA
     }
 }
 
+// wave_sum_d's value, bit for bit, without LDS permutes: the partners at
+// distances 32 and 16 by permlane swaps (a + b whichever of the two a lane is),
+// at 8 to 1 by row rotations (past distance d the values repeat with period
+// d, so lane i + d/2 holds what lane i ^ d/2 does).
+__device__ __forceinline__ double wave_sum_d_dpp(double v) {
+    typedef uint32_t u2 __attribute__((ext_vector_type(2)));
+    auto both = [](auto lo, auto hi) {
+        return __builtin_bit_cast(double, u2{lo[0], hi[0]}) + __builtin_bit_cast(double, u2{lo[1], hi[1]});
+    };
+    u2 w = __builtin_bit_cast(u2, v);
+    v = both(__builtin_amdgcn_permlane32_swap(w.x, w.x, false, false),
+             __builtin_amdgcn_permlane32_swap(w.y, w.y, false, false));
+    w = __builtin_bit_cast(u2, v);
+    v = both(__builtin_amdgcn_permlane16_swap(w.x, w.x, false, false),
+             __builtin_amdgcn_permlane16_swap(w.y, w.y, false, false));
+#define SRQ_ROR(ctrl)                                                                                  \
+    w = __builtin_bit_cast(u2, v);                                                                     \
+    v += __builtin_bit_cast(double, u2{(uint32_t)__builtin_amdgcn_update_dpp(0, (int)w.x, ctrl, 0xF, 0xF, false), \
+                                       (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w.y, ctrl, 0xF, 0xF, false)});
+    SRQ_ROR(0x128)
+    SRQ_ROR(0x124)
+    SRQ_ROR(0x122)
+    SRQ_ROR(0x121)
+#undef SRQ_ROR
+    return v;
+}
+
+// --------------------------------------------------------- short matrices
+// One batch row, rows of at most 2048 columns, at most 16 units per CU, one per
+// wave: a launch whose time is latency, not bytes.  Nothing is worth
+// streaming, so the kernel is one round of loads with no barrier: each wave
+// loads the whole of x (and of the norm weight), its unit's weights and its
+// epilogue's operands at once, normalises x itself and passes it through LDS
+// into the columns its lanes need.  All waves of a workgroup write the same
+// values to the same LDS words and each reads only after its own writes.  The
+// streaming kernel's staging and prefetch cursor cost such a launch two
+// barriers and some 14 KB of instructions.  Bits are the streaming kernel's:
+// the sum of squares adds in its order (pass p holds the columns that its
+// wave p stages), each row's dot is the same chain.
+// Measured, in a SmolLM2 decode step (Q8, 576 columns), streaming kernel -> here:
+// o and down 5.45 -> 2.7 us, q/k/v 5.7 -> 3.2, gate/up 5.9 -> 4.1; 64 greedy
+// tokens 58.2 -> 38.4 ms.  Up to 16 units per CU (3072 x 576 6.9 -> 5.1 us, 4096 x
+// 2048 Q4 6.4 -> 6.2); past that the streaming kernel's prefetch pays.
+constexpr int kShortWaves = 4;  // per workgroup
+
+// One unit's operands, loaded before x is needed.
+template <int FMT, int EPI, int NCH>
+struct ShortUnit {
+    using Ly = Lay<FMT, true>;
+    static constexpr int E = Ly::E, CW = Ly::CW, R = unit_rows_of<EPI>();
+    Unit t;
+    uint4 w[NCH][R];
+    float sc[NCH][R];
+    EpiOps o;
+    float resid;
+
+    __device__ __forceinline__ void load(const GemvArgs &A, int u, int lane) {
+        constexpr int SPC = FMT == SRQ_Q8 ? 16 : 32;  // scales per chunk
+        const int cols = (int)A.cols;
+        const int64_t rb = row_bytes(FMT, cols), sgroups = groups_of(cols);
+        const uint8_t *W = (const uint8_t *)A.values;
+        t = unit_rows<EPI>(A, u);
+#pragma unroll
+        for (int ch = 0; ch < NCH; ++ch) {
+            // a lane past the row end re-reads the row's start and meets zeros
+            const bool ok = ch * CW + lane * E < cols;
+            const uint32_t boff = ok ? (uint32_t)(ch * 1024 + lane * 16) : 0u;
+            const uint32_t soff = ok ? (uint32_t)(ch * SPC + lane / (FMT == SRQ_Q8 ? 4 : 2)) : 0u;
+#pragma unroll
+            for (int i = 0; i < R; ++i) {
+                w[ch][i] = ld_stream16(W + (uint64_t)(uint32_t)t.r[i] * (uint64_t)rb + boff);
+                sc[ch][i] = A.scales[(uint64_t)(uint32_t)t.r[i] * (uint64_t)sgroups + soff];
+            }
+        }
+        o = EpiOps{};
+        resid = 0.0f;
+        if constexpr (EPI == EPI_RESID) resid = A.residual[t.r[0]];
+        if constexpr (EPI == EPI_ROPE_KV) {
+            if (A.bias) o.bias0 = A.bias[t.r[0]], o.bias1 = A.bias[t.r[1]];
+            const float *cs = A.meta.rope_cs + (int64_t)A.row0 * A.head_dim + 2 * max(t.j, 0);
+            o.c = cs[0], o.s = cs[1];
+            o.kvoff = A.meta.kvoff[A.row0];
+        }
+    }
+
+    // The unit's dots with the staged x, and its stores.
+    __device__ __forceinline__ void finish(const GemvArgs &A, const float *xs, int lane) const {
+        bool wide = false;
+        float acc[R] = {}, v[R];
+#pragma unroll
+        for (int ch = 0; ch < NCH; ++ch) {
+            float xv[E];
+#pragma unroll
+            for (int q = 0; q < E / 4; ++q) {
+                const float4 f = *(const float4 *)(xs + ch * CW + q * 256 + lane * 4);
+                xv[4 * q] = f.x, xv[4 * q + 1] = f.y, xv[4 * q + 2] = f.z, xv[4 * q + 3] = f.w;
+                wide |= fmaxf(fmaxf(fabsf(f.x), fabsf(f.y)), fmaxf(fabsf(f.z), fabsf(f.w))) > kWideLimit;
+            }
+#pragma unroll
+            for (int i = 0; i < R; ++i) {
+                float wv[E];
+                decode16<FMT>(w[ch][i], wv);
+                float p = 0.0f;
+#pragma unroll
+                for (int e = 0; e < E; ++e) p = __builtin_fmaf(xv[e], wv[e], p);
+                if constexpr (FMT == SRQ_Q4) p *= 16.0f;  // exact: undo the /16 decode
+                acc[i] = __builtin_fmaf(p, sc[ch][i], acc[i]);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < R; ++i) v[i] = dpp_sum(acc[i]);
+        if (__any(wide)) {  // FP64 (M:4356-4382), as the streaming kernel's pass
+            const int64_t cols = A.cols, rb = row_bytes(FMT, cols), sgroups = groups_of(cols);
+#pragma unroll
+            for (int i = 0; i < R; ++i) {
+                const uint8_t *wr = (const uint8_t *)A.values + (int64_t)t.r[i] * rb;
+                double d = 0.0;
+                for (int64_t c = lane * 4; c < cols; c += 256) {
+                    double pp = 0.0;
+                    for (int e = 0; e < 4 && c + e < cols; ++e)
+                        pp += (double)xs[xidx<E, CW>((int)(c + e))] * (double)weight_at<FMT>(wr, c + e);
+                    d += pp * (double)A.scales[(int64_t)t.r[i] * sgroups + c / kBlock];
+                }
+                v[i] = (float)wave_sum_d(d);
+            }
+        }
+        if (lane == 0) store_unit<EPI, R>(A, t, A.y, v, resid, o);
+    }
+};
+
+__device__ __forceinline__ double sum4_sq(const float4 x) {
+    return (double)x.x * x.x + (double)x.y * x.y + (double)x.z * x.z + (double)x.w * x.w;
+}
+__device__ __forceinline__ float4 normed(const float4 x, float a, const float4 w) {
+    return make_float4(__fmul_rn(__fmul_rn(x.x, a), w.x), __fmul_rn(__fmul_rn(x.y, a), w.y),
+                       __fmul_rn(__fmul_rn(x.z, a), w.z), __fmul_rn(__fmul_rn(x.w, a), w.w));
+}
+
+template <int FMT, int EPI, bool NORM, int NCH>
+__global__ __launch_bounds__(64 * kShortWaves) void gemv_short_kernel(const GemvArgs A) {
+    using Ly = Lay<FMT, true>;
+    constexpr int E = Ly::E, CW = Ly::CW, NP = NCH * CW / 256;
+    __shared__ __attribute__((aligned(16))) float xs[NCH * CW];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int cols = (int)A.cols;
+    const int u = (int)blockIdx.x * kShortWaves + wave;
+    if (u >= unit_count<EPI>(A)) return;
+    float4 x[NP], nw[NP];
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+        const int c = p * 256 + lane * 4;
+        x[p] = c < cols ? *(const float4 *)(A.x + c) : make_float4(0.f, 0.f, 0.f, 0.f);
+        if (NORM) nw[p] = c < cols ? *(const float4 *)(A.norm_w + c) : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    ShortUnit<FMT, EPI, NCH> un;
+    un.load(A, u, lane);
+    if constexpr (NORM) {
+        // as stage_stream: f64 sums per wave of 256 columns, then in order
+        double tot = 0.0;
+#pragma unroll
+        for (int p = 0; p < NP; ++p) tot += wave_sum_d_dpp(sum4_sq(x[p]));
+        const float a = (float)(1.0 / sqrt(tot / (double)cols + A.norm_eps));
+#pragma unroll
+        for (int p = 0; p < NP; ++p) x[p] = normed(x[p], a, nw[p]);
+    }
+#pragma unroll
+    for (int p = 0; p < NP; ++p) *(float4 *)(xs + xidx<E, CW>(p * 256 + lane * 4)) = x[p];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+    un.finish(A, xs, lane);
+}
+
+// The same for rows of 2049 to 4096 columns, where every wave reading all of x
+// would cost as much as the weights: the eight waves of a workgroup stage x
+// together (one barrier, two with the norm), each then one unit.
+// Measured, in a Mistral-7B-width Q4 decode step, streaming kernel -> here: o
+// (4096 x 4096) 7.0 -> 4.7 us, q/k/v (6144 x 4096) 9.1 -> 7.4; alone, Q8 3072 x
+// 3072 5.5 -> 4.5 us a call.
+constexpr int kCoopCols = 4096;
+
+template <int FMT, int EPI, bool NORM, int NCH>
+__global__ __launch_bounds__(kStreamThreads) void gemv_coop_kernel(const GemvArgs A) {
+    using Ly = Lay<FMT, true>;
+    constexpr int E = Ly::E, CW = Ly::CW, NP = (NCH * CW + kStreamThreads * 4 - 1) / (kStreamThreads * 4);
+    __shared__ __attribute__((aligned(16))) float xs[NCH * CW];
+    __shared__ double ss[kStreamWaves];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int cols = (int)A.cols, units = unit_count<EPI>(A);
+    const int u = (int)blockIdx.x * kStreamWaves + wave;
+    float4 x[NP], nw[NP];
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+        const int c = (p * kStreamThreads + tid) * 4;
+        x[p] = c < cols ? *(const float4 *)(A.x + c) : make_float4(0.f, 0.f, 0.f, 0.f);
+        if (NORM) nw[p] = c < cols ? *(const float4 *)(A.norm_w + c) : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    ShortUnit<FMT, EPI, NCH> un;
+    un.load(A, min(u, units - 1), lane);
+    if constexpr (NORM) {
+        // stage_stream's sums: a thread's columns, its wave, the waves in order
+        double s = 0.0;
+#pragma unroll
+        for (int p = 0; p < NP; ++p) s += sum4_sq(x[p]);
+        s = wave_sum_d_dpp(s);
+        if (lane == 0) ss[wave] = s;
+        lds_barrier();
+        double tot = 0.0;
+#pragma unroll
+        for (int w = 0; w < kStreamWaves; ++w) tot += ss[w];
+        const float a = (float)(1.0 / sqrt(tot / (double)cols + A.norm_eps));
+#pragma unroll
+        for (int p = 0; p < NP; ++p) x[p] = normed(x[p], a, nw[p]);
+    }
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+        const int c = (p * kStreamThreads + tid) * 4;
+        if (c < NCH * CW) *(float4 *)(xs + xidx<E, CW>(c)) = x[p];
+    }
+    lds_barrier();
+    if (u < units) un.finish(A, xs, lane);
+}
+
+template <int FMT, int EPI, bool NORM>
+void launch_short(hipStream_t s, const GemvArgs &a, int64_t units, int nch) {
+    const dim3 grid((unsigned)((units + kShortWaves - 1) / kShortWaves));
+    const dim3 coop((unsigned)((units + kStreamWaves - 1) / kStreamWaves));
+    if constexpr (FMT == SRQ_Q8) {
+        switch (nch) {
+            case 1: gemv_short_kernel<FMT, EPI, NORM, 1><<<grid, 64 * kShortWaves, 0, s>>>(a); break;
+            case 2: gemv_short_kernel<FMT, EPI, NORM, 2><<<grid, 64 * kShortWaves, 0, s>>>(a); break;
+            case 3: gemv_coop_kernel<FMT, EPI, NORM, 3><<<coop, kStreamThreads, 0, s>>>(a); break;
+            default: gemv_coop_kernel<FMT, EPI, NORM, 4><<<coop, kStreamThreads, 0, s>>>(a); break;
+        }
+    } else {
+        if (nch == 1)
+            gemv_short_kernel<FMT, EPI, NORM, 1><<<grid, 64 * kShortWaves, 0, s>>>(a);
+        else
+            gemv_coop_kernel<FMT, EPI, NORM, 2><<<coop, kStreamThreads, 0, s>>>(a);
+    }
+}
+
 // Host-side launch parameters.
 int g_cus = 0;
 int device_cus() {
@@ -1177,6 +1437,15 @@ int launch_t(hipStream_t s, const GemvArgs &a) {
         if ((units / (blocks * kStreamWaves) + 1) * nch >= (1LL << 31))
             return fail(SRQ_EINVAL, "gemv: %lld x %lld exceeds the per-wave step limit", (long long)a.rows,
                         (long long)a.cols);
+        // One batch row of a short matrix: at most 16 units per CU.
+        if constexpr (NB == 1 && FMT != SRQ_F32) {
+            if (a.cols <= kCoopCols && units <= 16 * cap &&
+                ((((uintptr_t)a.x) | (NORM ? (uintptr_t)a.norm_w : 0)) & 15) == 0) {
+                launch_short<FMT, EPI, NORM>(s, a, units, nch);
+                SRQ_HIP(hipGetLastError());
+                return SRQ_OK;
+            }
+        }
         // One batch row: two units per step, so that their rows share each
         // read of the activations from LDS (Q4 reads 32 of them per 16
         // weight bytes).  Q8 pairs only one-row units: its two-row SwiGLU

@@ -932,6 +932,22 @@ __global__ __launch_bounds__(256) void attn_combine_heads_kernel(const AttnArgs 
     merge_splits<false>(A, part, nsplit, row, h0, nh, A.head_dim, used, cf, lse);
 }
 
+// The same for at most kChainSplits splits and head_dim 64 or 128: one wave per
+// (row, head), merge_wave's order (and so merge_splits' bits).  merge_splits
+// staged factors in LDS between barriers and brings 48 KB of unrolled code for
+// up to 1024 splits; a prefill row has a few.  256 rows x 32 heads at 2048
+// positions (4 splits): 14.8 -> 7.2 us.
+constexpr int kCombineWaves = 4;
+template <int HD>
+__global__ __launch_bounds__(64 * kCombineWaves) void attn_combine_wave_kernel(const AttnArgs A,
+                                                                               const float *__restrict__ part,
+                                                                               int nsplit, int split_len) {
+    const int row = blockIdx.x, h = blockIdx.y * kCombineWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (h >= A.heads) return;
+    const int len = A.meta.pos[row] + 1;
+    merge_wave<HD>(A, part, nsplit, row, h, min(nsplit, (len + split_len - 1) / split_len));
+}
+
 // ------------------------------------------------------------ prefill
 // Causal attention for prefill-sized steps on FP32 MFMA
 // (v_mfma_f32_16x16x4f32), flash style.  Workgroup (query tile, kv head,
@@ -1147,6 +1163,15 @@ int launch_attention(hipStream_t s, const AttnArgs &a, float *scratch, int32_t *
         else
             attn_flash_kernel<64><<<fg, 256, 0, s>>>(a, scratch, fsplit, ks);
         SRQ_HIP(hipGetLastError());
+        if (fsplit <= kChainSplits) {
+            const dim3 cg(a.n, (a.heads + kCombineWaves - 1) / kCombineWaves);
+            if (a.head_dim == 128)
+                attn_combine_wave_kernel<128><<<cg, 64 * kCombineWaves, 0, s>>>(a, scratch, fsplit, ks);
+            else
+                attn_combine_wave_kernel<64><<<cg, 64 * kCombineWaves, 0, s>>>(a, scratch, fsplit, ks);
+            SRQ_HIP(hipGetLastError());
+            return SRQ_OK;
+        }
         int nh = std::min(kMaxGroup, a.heads);
         while (a.heads % nh) --nh;
         attn_combine_heads_kernel<<<dim3(a.n, a.heads / nh), 256, 0, s>>>(a, scratch, fsplit, ks, nh);

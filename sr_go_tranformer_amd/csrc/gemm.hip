@@ -836,7 +836,10 @@ int launch_gemm(hipStream_t s, const GemmArgs &a, void *scratch, size_t scratch_
                      a.rope.dim % a.rope.head_dim || a.rope.kvdim % a.rope.head_dim ||
                      a.rows != (int64_t)a.rope.dim + 2 * (int64_t)a.rope.kvdim || a.y_stride != a.rows))
         return fail(SRQ_EINVAL, "gemm: RoPE/KV output needs rows = dim + 2*kvdim in whole heads and no other epilogue");
+    // (its LDS-direct loads want 16-byte aligned codes and scales, which a
+    // wrapped weight's pointers need not be)
     if (tall_ok(p, a.fmt, a.n, a.rows, a.cols) && scratch &&
+        ((((uintptr_t)a.values) | ((uintptr_t)a.scales)) & 15) == 0 &&
         scratch_bytes >= gemm_scratch_wanted(a.fmt, a.n, a.rows, a.cols)) {
         const size_t need = gemm_scratch_bytes(a.fmt, a.n, a.rows, a.cols);
         const size_t off = tall_offset(need + (p.slices == 1 ? (size_t)a.n * 4 : 0));

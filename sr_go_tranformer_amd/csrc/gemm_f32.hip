@@ -24,6 +24,10 @@ namespace {
 constexpr int BN = 128, BK = 32;
 constexpr int kStepBytes = BK * 4;  // one row of one step
 
+struct __attribute__((packed, aligned(4))) Loose {  // 16 bytes at any float
+    float v[4];
+};
+
 template <int BM>
 struct F32Tile {
     static constexpr int STAGE = (BM + BN) * kStepBytes;
@@ -31,8 +35,9 @@ struct F32Tile {
 };
 
 // Slices, partial and wflags as gemm_kernel (gemm.hip); kper counts K steps.
-// D: K steps the LDS ring holds.
-template <int BM, int D>
+// D: K steps the LDS ring holds.  DIRECT: operands 16-byte aligned, loaded
+// straight to LDS; otherwise they pass through registers.
+template <int BM, int D, bool DIRECT>
 __global__ __launch_bounds__(256, 1) void gemm_f32_kernel(const GemmArgs G, float *__restrict__ partial,
                                                           int32_t *__restrict__ wflags, const int kper) {
     typedef F32Tile<BM> T;
@@ -63,8 +68,13 @@ __global__ __launch_bounds__(256, 1) void gemm_f32_kernel(const GemmArgs G, floa
     auto load = [&](const int k, const uint32_t slot) {
         const int64_t off = (int64_t)(min(k, kend - 1) - kbeg) * kStepBytes;
 #pragma unroll
-        for (int j = 0; j < T::LOADS; ++j)
-            lds_load16(ring0 + slot + (uint32_t)((j * 4 + wave) * 1024), src[j] + off);
+        for (int j = 0; j < T::LOADS; ++j) {
+            const uint32_t at = slot + (uint32_t)((j * 4 + wave) * 1024);
+            if constexpr (DIRECT)
+                lds_load16(ring0 + at, src[j] + off);
+            else
+                *(Loose *)(&ring[0][0] + at + lane * 16) = *(const Loose *)(src[j] + off);
+        }
     };
 
     floatx4 acc[2][TN];
@@ -135,12 +145,15 @@ int launch_gemm_f32(hipStream_t s, const GemmArgs &a, float *partial, int32_t *w
     const int64_t wg32 = ft * ((a.n + 31) / 32);
     const int bm = a.n <= 32 || wg32 <= 256 ? 32 : 64;
     const dim3 grid((unsigned)((a.rows + BN - 1) / BN), (unsigned)((a.n + bm - 1) / bm), (unsigned)slices);
-    if (bm == 64)
-        gemm_f32_kernel<64, 3><<<grid, 256, 0, s>>>(a, partial, wflags, kper);
+    if ((((uintptr_t)a.x) | ((uintptr_t)a.values)) & 15)
+        gemm_f32_kernel<32, 3, false><<<dim3(grid.x, (unsigned)((a.n + 31) / 32), grid.z), 256, 0, s>>>(a, partial,
+                                                                                                       wflags, kper);
+    else if (bm == 64)
+        gemm_f32_kernel<64, 3, true><<<grid, 256, 0, s>>>(a, partial, wflags, kper);
     else if (kper > 4)
-        gemm_f32_kernel<32, 6><<<grid, 256, 0, s>>>(a, partial, wflags, kper);
+        gemm_f32_kernel<32, 6, true><<<grid, 256, 0, s>>>(a, partial, wflags, kper);
     else
-        gemm_f32_kernel<32, 3><<<grid, 256, 0, s>>>(a, partial, wflags, kper);
+        gemm_f32_kernel<32, 3, true><<<grid, 256, 0, s>>>(a, partial, wflags, kper);
     SRQ_HIP(hipGetLastError());
     return SRQ_OK;
 }

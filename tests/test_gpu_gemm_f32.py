@@ -2,6 +2,8 @@
 step to more than the LDS ring holds, split and unsplit, ragged rows and
 features, a row past the FP32 limit.  |err| <= (cols + 2) 2^-24 sum |x||w|: one
 rounding per addition of the longest chain."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -43,3 +45,49 @@ def test_f32_gemm(ex, rows, cols, ns):
         if first is None:
             first = got[:16]
         assert np.array_equal(got[:16].view(np.uint32), first.view(np.uint32)), n  # rows do not depend on n
+
+
+def test_f32_gemm_unaligned_rows(ex):
+    """Activations that start at any float, as a view into a larger buffer does:
+    the bits of the aligned call (F32, Q8 and Q4)."""
+    rng = oracle.RNG(3)
+    rows, cols, n = 300, 512, 150
+    dense = rng.fill_normal(rows * cols, 0.02).reshape(rows, cols)
+    x = rng.fill_normal(n * cols, 1.0).reshape(n, cols)
+    for fmt in (srq.F32, srq.Q8, srq.Q4):
+        w = srq.Weight.create(ex, dense, fmt)
+        for m in (1, 17, 32, n):
+            print("unaligned", fmt, m, flush=True)
+            want = srq.linear(ex, w, x[:m])
+            xb = ex.upload(np.concatenate([np.zeros(1, np.float32), x[:m].ravel()]))
+            yb = ex.empty(m * rows * 4)
+            srq.check(srq.lib().srq_linear(ex.h, yb.ptr, C.c_void_p(xb.ptr.value + 4), w.h, m))
+            got = yb.to_numpy(np.float32, (m, rows))
+            assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), (fmt, m)
+
+
+def test_wrapped_weights_at_any_float(ex):
+    """A wrapped weight whose scales (Q8, Q4) or values (F32) start off a 16-byte
+    boundary gives the aligned one's bits."""
+    rng = oracle.RNG(4)
+    rows, cols, n = 300, 512, 150
+    dense = rng.fill_normal(rows * cols, 0.02).reshape(rows, cols)
+    x = rng.fill_normal(n * cols, 1.0).reshape(n, cols)
+    one = np.zeros(1, np.float32)
+    for fmt in (srq.F32, srq.Q8, srq.Q4):
+        w = srq.Weight.create(ex, dense, fmt)
+        if fmt == srq.F32:
+            vb, off = ex.upload(np.concatenate([one, dense.ravel().astype(np.float32)])), 4
+            sp = None
+        else:
+            v, s = srq.pack(ex, dense, fmt)
+            vb, off = ex.upload(v), 0
+            sb = ex.upload(np.concatenate([one, np.asarray(s, np.float32).ravel()]))
+            sp = C.c_void_p(sb.ptr.value + 4)
+        h = C.c_void_p()
+        srq.check(srq.lib().srq_weight_wrap(fmt, rows, cols, C.c_void_p(vb.ptr.value + off), sp, C.byref(h)))
+        wrapped = srq.Weight(h)
+        for m in (17, 32, n):  # (one row of such F32 values takes the generic GEMV, another order)
+            print("wrapped", fmt, m, flush=True)
+            got, want = srq.linear(ex, wrapped, x[:m]), srq.linear(ex, w, x[:m])
+            assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), (fmt, m)

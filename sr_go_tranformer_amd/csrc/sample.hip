@@ -236,7 +236,11 @@ struct ChunkRed {
 // exp((v - vmax) / T) * 2^44 rounded, the quotient without a division per
 // value: y = RN(1/T), then two residual steps.  The first makes q faithful, the
 // second correctly rounds it (Markstein: a faithful q, an exact residual
-// and a correctly rounded reciprocal).  Temperatures far from 1 divide.
+// and a correctly rounded reciprocal).  Quotients that leave mass 0 return
+// before the steps, infinite ones among them (a large penalty takes values
+// past the f64 range), whose residuals would be NaN; past that test |v - vmax|
+// is at most 33 T.  Temperatures far from 1 divide.  32 x 128256 ids, per
+// call: 62.5 us, with a division per value 63.3.
 struct MassOf {
     double vmax, T, y;
     bool fast;
@@ -246,12 +250,13 @@ struct MassOf {
         double q;
         if (fast) {
             q = a * y;
+            if (!(q >= -33.0)) return 0;
             q = __builtin_fma(__builtin_fma(-T, q, a), y, q);
             q = __builtin_fma(__builtin_fma(-T, q, a), y, q);
         } else {
             q = a / T;
         }
-        if (q < -32.0) return 0;  // exp(-32) * 2^44 < 1/2
+        if (!(q >= -32.0)) return 0;  // exp(-32) * 2^44 < 1/2
         return (unsigned long long)(exp(q) * kFix + 0.5);
     }
 };

@@ -212,3 +212,21 @@ def test_sample_crowded_buckets(ex, vocab, spread):
         want, wst = oracle_rows(logits, t, k, p, rp, seeds, hist)
         assert np.array_equal(got, want), (t, k, p, got, want)
         assert np.array_equal(gst, wst)
+
+
+@pytest.mark.parametrize("t,rp", [(0.1, 1e308), (1e-3, 1e306), (1e-300, 1.1), (1e150, 1e300)])
+def test_sample_quotients_past_the_double_range(ex, t, rp):
+    """Penalties and temperatures that take a penalised value, or its distance
+    from the maximum over the temperature, past the f64 range: such a
+    candidate has mass 0, as exp of minus infinity does."""
+    print("past the double range", t, rp, flush=True)
+    rng = np.random.default_rng(5)
+    rows, vocab = 16, 900
+    logits = rng.normal(-1.0, 2.0, size=(rows, vocab)).astype(np.float32)
+    hist = [list(rng.choice(vocab, size=200, replace=False)) for _ in range(rows)]
+    seeds = rng.integers(0, 2**63, size=rows, dtype=np.uint64)
+    for k, p in ((0, 1.0), (0, 0.9), (40, 0.95)):
+        got, gst = run(ex, logits, srq.Sampling(t, k, p, rp), seeds, hist)
+        want, wst = oracle_rows(logits, t, k, p, rp, seeds, hist)
+        assert np.array_equal(got, want), (k, p, got, want)
+        assert np.array_equal(gst, wst)

@@ -149,10 +149,11 @@ int srq_linear_enqueue(srq_exec *e, float *y, const float *x, const srq_weight *
  * memory (code under HIP graph capture, serving loops that forbid
  * hipMalloc): srq_linear_enqueue -- the same kernels and bit-identical
  * results, stream-ordered on the executor without joining -- that allocates
- * nothing.  The GEMM path's split-K partial sums and wide-row flags go to a
- * fixed device array of SRQ_NOALLOC_SCRATCH_BYTES owned by the library (one
- * per GPU, held until the process ends) instead of the executor's
- * workspace.  A call whose plan needs more runs its rows in GEMM
+ * nothing.  The GEMM path's split-K partial sums and wide-row flags (and, of
+ * a call of many rows whose K is split, the split activations where they fit
+ * beside them) go to a fixed device array of SRQ_NOALLOC_SCRATCH_BYTES owned
+ * by the library (one per GPU, held until the process ends) instead of the
+ * executor's workspace.  A call whose plan needs more runs its rows in GEMM
  * sub-batches that fit the array, with the same bits (a row's GEMM result
  * does not depend on the rows beside it); with 64 MiB every n up to 1024
  * fits, and a plan that could not fit 17 rows would be rejected with

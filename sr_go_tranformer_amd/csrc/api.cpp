@@ -147,9 +147,10 @@ using namespace srq;
 // M:6062-6100).  Captured graphs point into a decoder's own workspace, so a
 // later step that grows the executor's workspace cannot invalidate them.
 struct Workspace {
-    DevBuf X, N, Q, A, T, H, W2, LOG, LOGC, meta, flags, ATT, ATTC, PLAN, SMP, SMPS;
+    DevBuf X, N, Q, A, T, H, W2, LOG, LOGC, meta, flags, planes, ATT, ATTC, PLAN, SMP, SMPS;
     void release_all() {
-        for (DevBuf *b : {&X, &N, &Q, &A, &T, &H, &W2, &LOG, &LOGC, &meta, &flags, &ATT, &ATTC, &PLAN, &SMP, &SMPS})
+        for (DevBuf *b : {&X, &N, &Q, &A, &T, &H, &W2, &LOG, &LOGC, &meta, &flags, &planes, &ATT, &ATTC, &PLAN, &SMP,
+                          &SMPS})
             release(*b);
     }
 };
@@ -344,38 +345,43 @@ size_t linear_scratch_bytes(const srq_weight &w, int32_t n, int32_t gemm_rows = 
     return n > gemm_rows && gemm_ok(w.fmt, w.cols) ? gemm_scratch_bytes(w.fmt, n, w.rows, w.cols) : 0;
 }
 
-// Workspace for launch_gemm: what it wants (split-K partial sums and, for
-// many rows, the activations' planes), or only what it needs where the
-// larger buffer cannot be had -- no memory, or a stream under capture, in
-// which nothing may be allocated and a call that needs no scratch still runs.
-int ensure_gemm(srq_exec *e, Workspace &ws, int fmt, int32_t n, int64_t rows, int64_t cols) {
-    const size_t wanted = gemm_scratch_wanted(fmt, n, rows, cols);
-    if (wanted <= ws.flags.n) return SRQ_OK;
-    const size_t need = gemm_scratch_bytes(fmt, n, rows, cols);
-    if (wanted > need) {
+// launch_gemm with the workspace's scratch and, for the calls that want them,
+// its buffer of activation planes.  Planes are optional (the bits are the
+// same without): a call goes without where the buffer cannot be had, and on
+// a stream under capture, so that a graph holds no pointer into a buffer that
+// a later call may grow -- the graph of an unsplit matrix, which needs no
+// scratch, holds no workspace pointer at all.
+int run_gemm(srq_exec *e, Workspace &ws, const GemmArgs &g) {
+    SRQ_CHECK(ensure(ws.flags, gemm_scratch_bytes(g.fmt, g.n, g.rows, g.cols), e->stream));
+    if (const size_t bytes = gemm_planes_bytes(g.fmt, g.n, g.rows, g.cols)) {
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
         SRQ_HIP(hipStreamIsCapturing(e->stream, &cap));
         if (cap == hipStreamCaptureStatusNone) {
-            if (ensure(ws.flags, wanted, e->stream) == SRQ_OK) return SRQ_OK;
+            if (ensure(ws.planes, bytes, e->stream) == SRQ_OK)
+                return launch_gemm(e->stream, g, ws.flags.p, ws.flags.n, ws.planes.p, ws.planes.n);
             (void)hipGetLastError();
             clear_error();
         }
     }
-    return ensure(ws.flags, need, e->stream);
+    return launch_gemm(e->stream, g, ws.flags.p, ws.flags.n, nullptr, 0);
 }
 
 // y[n x w.rows] = x . W^T for n rows through the GEMV (chunks of 8) or the
 // MFMA GEMM (n > gemm_rows, K multiple of 32), with optional fused RMSNorm.
-// fixed (non-null): the GEMM's scratch is that caller-provided buffer of
-// fixed_bytes instead of the workspace, which then never grows.
+// fixed (non-null): the GEMM's scratch and planes are in that caller-provided
+// buffer of fixed_bytes instead of the workspace, which then never grows.
 int run_linear(srq_exec *e, Workspace &ws, const srq_weight &w, const float *x, int32_t n, float *y, int64_t y_stride,
                const float *norm_w, double eps, const float *residual, int32_t gemm_rows = kLinearGemmRows,
                void *fixed = nullptr, size_t fixed_bytes = 0) {
     if (n > gemm_rows && gemm_ok(w.fmt, w.cols) && !norm_w) {
         GemmArgs g{w.fmt, w.values, w.scales, w.rows, w.cols, x, n, y, y_stride, residual, nullptr};
-        if (fixed) return launch_gemm(e->stream, g, fixed, fixed_bytes);
-        SRQ_CHECK(ensure_gemm(e, ws, w.fmt, n, w.rows, w.cols));
-        return launch_gemm(e->stream, g, ws.flags.p, ws.flags.n);
+        if (!fixed) return run_gemm(e, ws, g);
+        // The planes take what the partial sums leave; an unsplit matrix,
+        // which needs no scratch, leaves the buffer alone.
+        const size_t need = gemm_scratch_bytes(w.fmt, n, w.rows, w.cols), at = (need + 255) / 256 * 256;
+        const bool rest = need && at < fixed_bytes;
+        return launch_gemm(e->stream, g, fixed, fixed_bytes, rest ? (uint8_t *)fixed + at : nullptr,
+                           rest ? fixed_bytes - at : 0);
     }
     const int nb = gemv_max_rows(w.fmt, w.cols, norm_w != nullptr, 0);
     if (nb < 1) return fail(SRQ_EINVAL, "input width %lld exceeds the GEMV staging limit", (long long)w.cols);
@@ -1259,11 +1265,10 @@ int enqueue_layers(srq_exec *e, Workspace &ws, srq_model *m, srq_pool *pool, int
             // projection wrote it from its reduction.
             if (l == 0) SRQ_CHECK(launch_rmsnorm(e->stream, X, L.n1, N, n, (int32_t)d, c.norm_eps));
             // q/k/v GEMM with bias, RoPE and the KV write in its reduction.
-            SRQ_CHECK(ensure_gemm(e, ws, L.qkv.fmt, n, L.qkv.rows, L.qkv.cols));
             GemmArgs g{L.qkv.fmt, L.qkv.values, L.qkv.scales, L.qkv.rows, L.qkv.cols, N, n, W2, d + 2 * kd,
                        nullptr, nullptr};
             g.rope = GemmRope{Q, L.bias, (int32_t)d, (int32_t)kd, m->hd, m->cos_t, m->sin_t, meta};
-            SRQ_CHECK(launch_gemm(e->stream, g, ws.flags.p, ws.flags.n));
+            SRQ_CHECK(run_gemm(e, ws, g));
         }
         AttnArgs at{};
         at.q = Q;
@@ -1282,12 +1287,11 @@ int enqueue_layers(srq_exec *e, Workspace &ws, srq_model *m, srq_pool *pool, int
             SRQ_CHECK(run_linear(e, ws, L.o, A, n, X, d, nullptr, 0.0, X, kStepGemmRows));
         } else {
             // with RMSNorm(X, n2) -> N in its reduction
-            SRQ_CHECK(ensure_gemm(e, ws, L.o.fmt, n, L.o.rows, L.o.cols));
             GemmArgs g{L.o.fmt, L.o.values, L.o.scales, L.o.rows, L.o.cols, A, n, X, d, X, nullptr};
             g.norm_w = L.n2;
             g.norm_eps = c.norm_eps;
             g.norm_out = N;
-            SRQ_CHECK(launch_gemm(e->stream, g, ws.flags.p, ws.flags.n));
+            SRQ_CHECK(run_gemm(e, ws, g));
         }
         if (!use_gemm) {
             for (int32_t r0 = 0; r0 < n; r0 += nbg) {
@@ -1310,21 +1314,19 @@ int enqueue_layers(srq_exec *e, Workspace &ws, srq_model *m, srq_pool *pool, int
         } else {
             // gate/up GEMM with SwiGLU in its split-K reduction (W2 is only
             // a temporary when K is not split).
-            SRQ_CHECK(ensure_gemm(e, ws, L.gu.fmt, n, L.gu.rows, L.gu.cols));
             GemmArgs g{L.gu.fmt, L.gu.values, L.gu.scales, L.gu.rows, L.gu.cols, N, n, W2, 2 * H, nullptr, Hh};
-            SRQ_CHECK(launch_gemm(e->stream, g, ws.flags.p, ws.flags.n));
+            SRQ_CHECK(run_gemm(e, ws, g));
         }
         // down + residual (M:6415-6417).
         if (!use_gemm || l + 1 == c.layers) {
             SRQ_CHECK(run_linear(e, ws, L.down, Hh, n, X, d, nullptr, 0.0, X, kStepGemmRows));
         } else {
             // with the next layer's RMSNorm(X, n1) -> N in its reduction
-            SRQ_CHECK(ensure_gemm(e, ws, L.down.fmt, n, L.down.rows, L.down.cols));
             GemmArgs g{L.down.fmt, L.down.values, L.down.scales, L.down.rows, L.down.cols, Hh, n, X, d, X, nullptr};
             g.norm_w = m->L[l + 1].n1;
             g.norm_eps = c.norm_eps;
             g.norm_out = N;
-            SRQ_CHECK(launch_gemm(e->stream, g, ws.flags.p, ws.flags.n));
+            SRQ_CHECK(run_gemm(e, ws, g));
         }
         if (cancel && (l + 1) % kEventEvery == 0)
             SRQ_HIP(hipEventRecord(e->layer_done[(l / kEventEvery) % kSlots], e->stream));

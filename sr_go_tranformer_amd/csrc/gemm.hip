@@ -786,7 +786,7 @@ size_t gemm_scratch_bytes(int fmt, int32_t n, int64_t rows, int64_t cols) {
     return (size_t)p.slices * (size_t)n * ((size_t)rows + 1) * 4;
 }
 
-// Whether a call of n rows takes the tall tiles (gemm_tall.hip), given scratch
+// Whether a call of n rows takes the tall tiles (gemm_tall.hip), given memory
 // for its planes.  They cost one more launch (about 4 us with its gap).
 // Q4, whose 64-row tiles here convert more per MFMA, gains from 33 rows on
 // (28672 x 4096 at 40 rows 90 -> 57 us, 512 x 512 19.7 -> 14.6 us).  Q8 gains
@@ -802,20 +802,21 @@ static bool tall_ok(const GemmPlan &p, int fmt, int32_t n, int64_t rows, int64_t
     return macs >= 3.2e9 || (n > 128 && macs >= 1.4e9);
 }
 
-// Layout: partial sums, their wide-row flags, then (256-aligned) the tall
-// tiles' flags and planes.
-static size_t tall_offset(size_t need) { return (need + 255) / 256 * 256; }
-
-size_t gemm_scratch_wanted(int fmt, int32_t n, int64_t rows, int64_t cols) {
-    const size_t need = gemm_scratch_bytes(fmt, n, rows, cols);
-    if (n <= 0 || rows <= 0 || !gemm_ok(fmt, cols)) return need;
-    const GemmPlan p = plan_gemm(fmt, n, rows, cols);
-    if (!tall_ok(p, fmt, n, rows, cols)) return need;
-    const TallPlan t = tall_plan(n, rows, p.slices);
-    return tall_offset(need + (p.slices == 1 ? (size_t)n * 4 : 0)) + tall_plane_bytes(t, n, cols);
+// Layout: the wide-row flags of an unsplit call (a split one's are in its
+// scratch), then the planes.
+static size_t plane_offset(const GemmPlan &p, int32_t n) {
+    return p.slices == 1 ? ((size_t)n * 4 + 255) / 256 * 256 : 0;
 }
 
-int launch_gemm(hipStream_t s, const GemmArgs &a, void *scratch, size_t scratch_bytes) {
+size_t gemm_planes_bytes(int fmt, int32_t n, int64_t rows, int64_t cols) {
+    if (n <= 0 || rows <= 0 || !gemm_ok(fmt, cols)) return 0;
+    const GemmPlan p = plan_gemm(fmt, n, rows, cols);
+    if (!tall_ok(p, fmt, n, rows, cols)) return 0;
+    return plane_offset(p, n) + tall_plane_bytes(tall_plan(n, rows, p.slices), n, cols);
+}
+
+int launch_gemm(hipStream_t s, const GemmArgs &a, void *scratch, size_t scratch_bytes, void *planes,
+                size_t planes_bytes) {
     if (a.n <= 0 || a.rows <= 0) return SRQ_OK;
     if (!gemm_ok(a.fmt, a.cols)) return fail(SRQ_EINVAL, "gemm: cols=%lld not a multiple of %d", (long long)a.cols, BK);
     const GemmPlan p = plan_gemm(a.fmt, a.n, a.rows, a.cols);
@@ -838,14 +839,12 @@ int launch_gemm(hipStream_t s, const GemmArgs &a, void *scratch, size_t scratch_
         return fail(SRQ_EINVAL, "gemm: RoPE/KV output needs rows = dim + 2*kvdim in whole heads and no other epilogue");
     // (its LDS-direct loads want 16-byte aligned codes and scales, which a
     // wrapped weight's pointers need not be)
-    if (tall_ok(p, a.fmt, a.n, a.rows, a.cols) && scratch &&
+    if (planes && tall_ok(p, a.fmt, a.n, a.rows, a.cols) &&
         ((((uintptr_t)a.values) | ((uintptr_t)a.scales)) & 15) == 0 &&
-        scratch_bytes >= gemm_scratch_wanted(a.fmt, a.n, a.rows, a.cols)) {
-        const size_t need = gemm_scratch_bytes(a.fmt, a.n, a.rows, a.cols);
-        const size_t off = tall_offset(need + (p.slices == 1 ? (size_t)a.n * 4 : 0));
-        if (!wflags) wflags = (int32_t *)scratch;
-        SRQ_CHECK(launch_gemm_tall(s, a, tall_plan(a.n, a.rows, p.slices), (uint8_t *)scratch + off, partial, wflags,
-                                   p.slices, p.kper));
+        planes_bytes >= gemm_planes_bytes(a.fmt, a.n, a.rows, a.cols)) {
+        if (!wflags) wflags = (int32_t *)planes;
+        SRQ_CHECK(launch_gemm_tall(s, a, tall_plan(a.n, a.rows, p.slices), (uint8_t *)planes + plane_offset(p, a.n),
+                                   partial, wflags, p.slices, p.kper));
     } else if (a.fmt == SRQ_F32) {
         SRQ_CHECK(launch_gemm_f32(s, a, partial, wflags, p.slices, p.kper));
     } else if (p.bm == 16) {

@@ -161,12 +161,14 @@ struct GemmArgs {
 // y = x . W^T (+ residual) on MFMA.  Rows holding a wide |x| are computed
 // in FP64.  scratch: gemm_scratch_bytes(fmt, n, rows, cols) bytes of device
 // memory for split-K partial sums (0: none needed).
-int launch_gemm(hipStream_t s, const GemmArgs &a, void *scratch, size_t scratch_bytes);
+// planes: with gemm_planes_bytes (0: no use for them) bytes of device memory,
+// 256-byte aligned, a call of many rows splits its activations once
+// (gemm_tall.hip); with less or null it runs the smaller tiles.  Either way
+// the results have the same bits.
+int launch_gemm(hipStream_t s, const GemmArgs &a, void *scratch, size_t scratch_bytes, void *planes,
+                size_t planes_bytes);
 size_t gemm_scratch_bytes(int fmt, int32_t n, int64_t rows, int64_t cols);
-// With this much scratch a call of many rows also keeps its activations'
-// split planes there (gemm_tall.hip); with less it runs the smaller tiles.
-// Either way the results have the same bits.
-size_t gemm_scratch_wanted(int fmt, int32_t n, int64_t rows, int64_t cols);
+size_t gemm_planes_bytes(int fmt, int32_t n, int64_t rows, int64_t cols);
 bool gemm_ok(int fmt, int64_t cols);
 
 // ------------------------------------------------------------------ glue

@@ -19,6 +19,7 @@
 #include <vector>
 
 #include "srq_internal.h"
+#include "workspace.h"
 
 // Scratch of srq_linear_noalloc (split-K partial sums and wide-row flags of
 // the GEMM path): a fixed array of the code object, one copy per GPU, held
@@ -70,32 +71,25 @@ int prepare_device(int device) {
     return SRQ_OK;
 }
 
-struct DevBuf {
-    void *p = nullptr;
-    size_t n = 0;
+// Device memory calls of workspace.h.
+struct DeviceMem {
+    hipStream_t s;
+    hipError_t err = hipSuccess;  // of the last call that failed
+    size_t bytes = 0;             // of the last allocation that failed
+    bool check(hipError_t e) {
+        if (e != hipSuccess) err = e;
+        return e == hipSuccess;
+    }
+    bool alloc(void **p, size_t n) {
+        if (check(hipMalloc(p, n))) return true;
+        (void)hipGetLastError();
+        bytes = n;
+        return false;
+    }
+    bool release(void *p) { return check(hipFree(p)); }
+    bool sync() { return check(hipStreamSynchronize(s)); }
+    bool out_of_memory() const { return err == hipErrorOutOfMemory; }
 };
-
-// Grows b to at least `bytes`.  A buffer that has to grow again takes half
-// as much again as it held, so steps whose shapes creep up (the attention
-// scratch gains a split every 64 positions) reallocate -- a stream
-// synchronisation, a free and an allocation -- a logarithmic number of times.
-int ensure(DevBuf &b, size_t bytes, hipStream_t s) {
-    if (bytes <= b.n) return SRQ_OK;
-    size_t want = std::max(bytes, (size_t)256);
-    if (b.p) {
-        want = std::max(want, b.n + b.n / 2);
-        SRQ_HIP(hipStreamSynchronize(s));
-        SRQ_HIP(hipFree(b.p));
-        b.p = nullptr;
-        b.n = 0;
-    }
-    if (hipMalloc(&b.p, want) != hipSuccess) {
-        b.p = nullptr;
-        return fail(SRQ_ENOMEM, "device allocation of %zu bytes failed", want);
-    }
-    b.n = want;
-    return SRQ_OK;
-}
 
 void release(DevBuf &b) {
     if (b.p) (void)hipFree(b.p);
@@ -147,11 +141,12 @@ using namespace srq;
 // M:6062-6100).  Captured graphs point into a decoder's own workspace, so a
 // later step that grows the executor's workspace cannot invalidate them.
 struct Workspace {
-    DevBuf X, N, Q, A, T, H, W2, LOG, LOGC, meta, flags, planes, ATT, ATTC, PLAN, SMP, SMPS;
+    DevBuf X, N, Q, A, T, H, W2, LOG, LOGC, meta, flags, ATT, ATTC, PLAN, SMP, SMPS;
+    OptionalBuf planes;  // split activations of many-row GEMMs
     void release_all() {
-        for (DevBuf *b : {&X, &N, &Q, &A, &T, &H, &W2, &LOG, &LOGC, &meta, &flags, &planes, &ATT, &ATTC, &PLAN, &SMP,
-                          &SMPS})
+        for (DevBuf *b : {&X, &N, &Q, &A, &T, &H, &W2, &LOG, &LOGC, &meta, &flags, &ATT, &ATTC, &PLAN, &SMP, &SMPS})
             release(*b);
+        release(planes);
     }
 };
 
@@ -250,6 +245,14 @@ int check_err_flag(srq_exec *e, int code, const char *what) {
         return fail(code, "%s", what);
     }
     return SRQ_OK;
+}
+
+// Grows b, a buffer of ws, to at least `bytes`.
+int ensure(Workspace &ws, DevBuf &b, size_t bytes, hipStream_t s) {
+    DeviceMem mem{s};
+    if (grow_or_give_back(b, bytes, ws.planes, mem)) return SRQ_OK;
+    if (mem.bytes) return fail(SRQ_ENOMEM, "device allocation of %zu bytes failed", mem.bytes);
+    return fail(SRQ_EDEVICE, "workspace growth: %s", hipGetErrorString(mem.err));
 }
 
 // Error word of a packer call that joins before it returns: pinned host
@@ -352,15 +355,14 @@ size_t linear_scratch_bytes(const srq_weight &w, int32_t n, int32_t gemm_rows = 
 // a later call may grow -- the graph of an unsplit matrix, which needs no
 // scratch, holds no workspace pointer at all.
 int run_gemm(srq_exec *e, Workspace &ws, const GemmArgs &g) {
-    SRQ_CHECK(ensure(ws.flags, gemm_scratch_bytes(g.fmt, g.n, g.rows, g.cols), e->stream));
+    SRQ_CHECK(ensure(ws, ws.flags, gemm_scratch_bytes(g.fmt, g.n, g.rows, g.cols), e->stream));
     if (const size_t bytes = gemm_planes_bytes(g.fmt, g.n, g.rows, g.cols)) {
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
         SRQ_HIP(hipStreamIsCapturing(e->stream, &cap));
         if (cap == hipStreamCaptureStatusNone) {
-            if (ensure(ws.planes, bytes, e->stream) == SRQ_OK)
+            DeviceMem mem{e->stream};
+            if (grow_optional(ws.planes, bytes, mem))
                 return launch_gemm(e->stream, g, ws.flags.p, ws.flags.n, ws.planes.p, ws.planes.n);
-            (void)hipGetLastError();
-            clear_error();
         }
     }
     return launch_gemm(e->stream, g, ws.flags.p, ws.flags.n, nullptr, 0);
@@ -1348,21 +1350,21 @@ int enqueue_head(srq_exec *e, Workspace &ws, srq_model *m, const float *rows, in
 int ensure_workspace(srq_exec *e, Workspace &ws, srq_model *m, int32_t n, int32_t sessions, int32_t max_len) {
     const int64_t d = m->c.dim, kd = m->kvdim, H = m->c.hidden, V = m->c.vocab;
     const size_t nd = (size_t)n * d * 4;
-    SRQ_CHECK(ensure(ws.X, nd, e->stream));
-    SRQ_CHECK(ensure(ws.N, nd, e->stream));
-    SRQ_CHECK(ensure(ws.Q, nd, e->stream));
-    SRQ_CHECK(ensure(ws.A, nd, e->stream));
-    SRQ_CHECK(ensure(ws.T, (size_t)std::max<int64_t>(n, sessions) * d * 4, e->stream));
-    SRQ_CHECK(ensure(ws.H, (size_t)n * H * 4, e->stream));
-    SRQ_CHECK(ensure(ws.W2, (size_t)n * std::max<int64_t>(d + 2 * kd, 2 * H) * 4, e->stream));
-    SRQ_CHECK(ensure(ws.LOGC, (size_t)sessions * V * 4, e->stream));
-    SRQ_CHECK(ensure(ws.LOG, (size_t)sessions * V * 4, e->stream));
-    SRQ_CHECK(ensure(ws.ATT, attention_scratch_bytes(n, m->c.heads, m->hd, max_len), e->stream));
-    SRQ_CHECK(ensure(ws.PLAN, (size_t)n * 8 + (size_t)n * m->hd * 4, e->stream));
+    SRQ_CHECK(ensure(ws, ws.X, nd, e->stream));
+    SRQ_CHECK(ensure(ws, ws.N, nd, e->stream));
+    SRQ_CHECK(ensure(ws, ws.Q, nd, e->stream));
+    SRQ_CHECK(ensure(ws, ws.A, nd, e->stream));
+    SRQ_CHECK(ensure(ws, ws.T, (size_t)std::max<int64_t>(n, sessions) * d * 4, e->stream));
+    SRQ_CHECK(ensure(ws, ws.H, (size_t)n * H * 4, e->stream));
+    SRQ_CHECK(ensure(ws, ws.W2, (size_t)n * std::max<int64_t>(d + 2 * kd, 2 * H) * 4, e->stream));
+    SRQ_CHECK(ensure(ws, ws.LOGC, (size_t)sessions * V * 4, e->stream));
+    SRQ_CHECK(ensure(ws, ws.LOG, (size_t)sessions * V * 4, e->stream));
+    SRQ_CHECK(ensure(ws, ws.ATT, attention_scratch_bytes(n, m->c.heads, m->hd, max_len), e->stream));
+    SRQ_CHECK(ensure(ws, ws.PLAN, (size_t)n * 8 + (size_t)n * m->hd * 4, e->stream));
     // Attention merge counters start at zero; the kernels leave them zero.
     const size_t cbytes = (size_t)n * m->c.heads * 4;
     if (cbytes > ws.ATTC.n) {
-        SRQ_CHECK(ensure(ws.ATTC, cbytes, e->stream));
+        SRQ_CHECK(ensure(ws, ws.ATTC, cbytes, e->stream));
         SRQ_CHECK(launch_zero(e->stream, as<int32_t>(ws.ATTC), (int64_t)(ws.ATTC.n / 4)));
     }
     return SRQ_OK;
@@ -1386,7 +1388,7 @@ extern "C" int srq_step(srq_exec *e, srq_model *m, int32_t sessions, srq_cache *
     SRQ_CHECK(ensure_workspace(e, ws, m, n, sessions, max_pos));
     const int32_t pt_stride = (m->c.context + kPageTokens - 1) / kPageTokens;
     const size_t words = meta_words(n, sessions, pt_stride);
-    SRQ_CHECK(ensure(ws.meta, words * 4, e->stream));
+    SRQ_CHECK(ensure(ws, ws.meta, words * 4, e->stream));
     SRQ_CHECK(ensure_host_meta(e, words));
     SRQ_HIP(hipStreamSynchronize(e->stream));  // the pinned staging may still feed a copy
 
@@ -1463,7 +1465,7 @@ extern "C" int srq_argmax(srq_exec *e, const float *logits, int32_t rows, int32_
     if (!e || !logits || !ids) return fail(SRQ_EINVAL, "null pointer");
     if (rows < 1 || vocab < 1) return fail(SRQ_EINVAL, "empty logits");
     DeviceGuard g(e->device);
-    SRQ_CHECK(ensure(e->ws.flags, sizeof(int32_t) * (size_t)rows, e->stream));
+    SRQ_CHECK(ensure(e->ws, e->ws.flags, sizeof(int32_t) * (size_t)rows, e->stream));
     SRQ_CHECK(launch_argmax(e->stream, logits, rows, vocab, as<int32_t>(e->ws.flags), e->d_err));
     SRQ_HIP(hipMemcpyAsync(ids, e->ws.flags.p, sizeof(int32_t) * rows, hipMemcpyDeviceToHost, e->stream));
     return check_err_flag(e, SRQ_ENONFINITE, "non-finite HF logits");
@@ -1488,8 +1490,8 @@ extern "C" int srq_sample(srq_exec *e, const float *logits, int32_t rows, const 
     // on the device the history, in the pinned buffer the results
     // [ids: rows][errors: rows] (the advanced states replace rng there)
     const size_t words = (size_t)rows * 5 + hist_words;
-    SRQ_CHECK(ensure(ws.SMP, words * 4, e->stream));
-    SRQ_CHECK(ensure(ws.SMPS, sample_scratch_bytes(rows, vocab), e->stream));
+    SRQ_CHECK(ensure(ws, ws.SMP, words * 4, e->stream));
+    SRQ_CHECK(ensure(ws, ws.SMPS, sample_scratch_bytes(rows, vocab), e->stream));
     int32_t *d = as<int32_t>(ws.SMP);
     uint64_t *d_rng = (uint64_t *)d;
     int32_t *d_blk = d + 2 * rows, *d_hl = d + 3 * rows, *d_rows = d + 4 * rows;

@@ -36,7 +36,11 @@ struct F32Tile {
 
 // Slices, partial and wflags as gemm_kernel (gemm.hip); kper counts K steps.
 // D: K steps the LDS ring holds.  DIRECT: operands 16-byte aligned, loaded
-// straight to LDS; otherwise they pass through registers.
+// straight to LDS.  Otherwise (D = 2) they pass through registers: step k + 1
+// is in flight during the MFMAs of step k and stored after them (loaded and
+// stored before them, every step waited for memory: activations off by one
+// float, 49152 x 576 at 32 / 1000 rows 46 -> 29 / 724 -> 502 us, 3072 x 576 at
+// 129 rows 15.8 -> 14.5 us).
 template <int BM, int D, bool DIRECT>
 __global__ __launch_bounds__(256, 1) void gemm_f32_kernel(const GemmArgs G, float *__restrict__ partial,
                                                           int32_t *__restrict__ wflags, const int kper) {
@@ -65,16 +69,22 @@ __global__ __launch_bounds__(256, 1) void gemm_f32_kernel(const GemmArgs G, floa
         src[j] = (const uint8_t *)(row + (int64_t)kbeg * BK) + chunk * 16;
     }
     const uint32_t ring0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)&ring[0][0];
+    auto step_off = [&](const int k) { return (int64_t)(min(k, kend - 1) - kbeg) * kStepBytes; };
     auto load = [&](const int k, const uint32_t slot) {
-        const int64_t off = (int64_t)(min(k, kend - 1) - kbeg) * kStepBytes;
 #pragma unroll
-        for (int j = 0; j < T::LOADS; ++j) {
-            const uint32_t at = slot + (uint32_t)((j * 4 + wave) * 1024);
-            if constexpr (DIRECT)
-                lds_load16(ring0 + at, src[j] + off);
-            else
-                *(Loose *)(&ring[0][0] + at + lane * 16) = *(const Loose *)(src[j] + off);
-        }
+        for (int j = 0; j < T::LOADS; ++j)
+            lds_load16(ring0 + slot + (uint32_t)((j * 4 + wave) * 1024), src[j] + step_off(k));
+    };
+    Loose held[DIRECT ? 1 : T::LOADS];
+    auto fetch = [&](const int k) {
+#pragma unroll
+        for (int j = 0; j < T::LOADS; ++j) held[j] = *(const Loose *)(src[j] + step_off(k));
+    };
+    auto put = [&](const uint32_t slot) {
+#pragma unroll
+        for (int j = 0; j < T::LOADS; ++j)
+            *(floatx4 *)(&ring[0][0] + slot + (j * 4 + wave) * 1024 + lane * 16) =
+                floatx4{held[j].v[0], held[j].v[1], held[j].v[2], held[j].v[3]};
     };
 
     floatx4 acc[2][TN];
@@ -83,8 +93,14 @@ __global__ __launch_bounds__(256, 1) void gemm_f32_kernel(const GemmArgs G, floa
 #pragma unroll
         for (int j = 0; j < TN; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
     float amax[2] = {0.f, 0.f};
+    if constexpr (DIRECT) {
 #pragma unroll
-    for (int d = 0; d < D - 1; ++d) load(kbeg + d, (uint32_t)(d * T::STAGE));
+        for (int d = 0; d < D - 1; ++d) load(kbeg + d, (uint32_t)(d * T::STAGE));
+    } else {
+        fetch(kbeg);
+        put(0);
+        fetch(kbeg + 1);
+    }
     // operand chunks 2gq and 2gq + 1 of row li of a tile
     const int rd[2] = {((2 * gq) ^ (li & 7)) * 16 + li * kStepBytes, ((2 * gq + 1) ^ (li & 7)) * 16 + li * kStepBytes};
     uint32_t cur = 0, fill = (D - 1) * T::STAGE;
@@ -92,9 +108,9 @@ __global__ __launch_bounds__(256, 1) void gemm_f32_kernel(const GemmArgs G, floa
         // Step k has landed when at most the D - 2 later steps' loads are
         // outstanding; past the barrier every wave's share of it has, and no
         // wave reads step k - 1, whose slot the next load fills.
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((D - 2) * T::LOADS) : "memory");
+        if constexpr (DIRECT) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((D - 2) * T::LOADS) : "memory");
         lds_barrier();
-        load(k + D - 1, fill);
+        if constexpr (DIRECT) load(k + D - 1, fill);
         const uint8_t *as = &ring[0][0] + cur, *bs = as + BM * kStepBytes;
         float af[2][8], bf[TN][8];
 #pragma unroll
@@ -122,6 +138,10 @@ __global__ __launch_bounds__(256, 1) void gemm_f32_kernel(const GemmArgs G, floa
                     acc[tm][tn] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[tm][s], bf[tn][s], acc[tm][tn], 0, 0, 0);
                 amax[tm] = fmaxf(amax[tm], fabsf(af[tm][s]));
             }
+        if constexpr (!DIRECT) {
+            put(fill);
+            fetch(k + 2);
+        }
         cur = cur == (D - 1) * T::STAGE ? 0 : cur + T::STAGE;
         fill = fill == (D - 1) * T::STAGE ? 0 : fill + T::STAGE;
     }
@@ -145,9 +165,11 @@ int launch_gemm_f32(hipStream_t s, const GemmArgs &a, float *partial, int32_t *w
     const int64_t wg32 = ft * ((a.n + 31) / 32);
     const int bm = a.n <= 32 || wg32 <= 256 ? 32 : 64;
     const dim3 grid((unsigned)((a.rows + BN - 1) / BN), (unsigned)((a.n + bm - 1) / bm), (unsigned)slices);
-    if ((((uintptr_t)a.x) | ((uintptr_t)a.values)) & 15)
-        gemm_f32_kernel<32, 3, false><<<dim3(grid.x, (unsigned)((a.n + 31) / 32), grid.z), 256, 0, s>>>(a, partial,
-                                                                                                       wflags, kper);
+    const bool loose = (((uintptr_t)a.x) | ((uintptr_t)a.values)) & 15;
+    if (loose && bm == 64)
+        gemm_f32_kernel<64, 2, false><<<grid, 256, 0, s>>>(a, partial, wflags, kper);
+    else if (loose)
+        gemm_f32_kernel<32, 2, false><<<grid, 256, 0, s>>>(a, partial, wflags, kper);
     else if (bm == 64)
         gemm_f32_kernel<64, 3, true><<<grid, 256, 0, s>>>(a, partial, wflags, kper);
     else if (kper > 4)

@@ -66,6 +66,35 @@ def test_f32_gemm_unaligned_rows(ex):
             assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), (fmt, m)
 
 
+@pytest.mark.parametrize("rows,cols,ns", [
+    (3, 32, (17, 33)),           # one step: what follows it is loaded again, never used
+    (130, 64, (32, 65, 300)),    # two steps
+    (1000, 608, (17, 97)),       # split K, a shorter last slice
+    (33000, 224, (40, 66)),      # not split, 64-row tiles
+])
+def test_f32_steps_through_registers(ex, rows, cols, ns):
+    """F32 operands off a 16-byte boundary (activations, then also the values):
+    the aligned call's bits, at the edges of the steps and tiles."""
+    rng = oracle.RNG(rows + cols)
+    dense = np.resize(rng.fill_normal(1 << 16, 0.02), rows * cols).reshape(rows, cols).astype(np.float32)
+    w = srq.Weight.create(ex, dense, srq.F32)
+    one = np.zeros(1, np.float32)
+    vb = ex.upload(np.concatenate([one, dense.ravel()]))
+    h = C.c_void_p()
+    srq.check(srq.lib().srq_weight_wrap(srq.F32, rows, cols, C.c_void_p(vb.ptr.value + 4), None, C.byref(h)))
+    wrapped = srq.Weight(h)
+    for n in ns:
+        print("f32 registers", rows, cols, n, flush=True)
+        x = np.resize(rng.fill_normal(1 << 15, 1.0), n * cols).reshape(n, cols).copy()
+        x[n - 1, cols // 2] = 3e34
+        want = srq.linear(ex, w, x)
+        xb = ex.upload(np.concatenate([one, x.ravel()]))
+        for weights in (w, wrapped):
+            yb = ex.empty(n * rows * 4)
+            srq.check(srq.lib().srq_linear(ex.h, yb.ptr, C.c_void_p(xb.ptr.value + 4), weights.h, n))
+            assert np.array_equal(yb.to_numpy(np.uint32, (n, rows)), want.view(np.uint32)), n
+
+
 def test_wrapped_weights_at_any_float(ex):
     """A wrapped weight whose scales (Q8, Q4) or values (F32) start off a 16-byte
     boundary gives the aligned one's bits."""

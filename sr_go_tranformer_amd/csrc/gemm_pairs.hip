@@ -22,6 +22,7 @@
 // 28672 x 4096 54 -> 42 us, 6144 x 4096 (13) 19.6 -> 17.4 us, 512 x 512 (4)
 // 9.6 -> 8.4 us.  What bounds it: the per-block work of a wave (code
 // conversion, the activation split, LDS) at 3-4 TB/s of weights.
+#include <climits>
 #include <utility>
 
 #include "gemm_x3.h"
@@ -294,15 +295,31 @@ void launch_exact(const PairCall &c) {
     }
 }
 
-// Blocks run by chunks of ku, each chunk's first loads counted as two.
-int chunk_cost(int kper, int ku) { return (kper + ku - 1) / ku * (ku + 2); }
+// Blocks per chunk of a slice of kper > 16 blocks: the cheapest, counting the
+// blocks of a short last chunk (it runs them all) and two for each chunk's
+// first loads.  Nine and ten are there for slices just past 16 blocks: in
+// chunks of 12, 17 or 18 blocks ran 24 (8192 features in four slices, 24 rows,
+// Q4: 17 / 18 / 19 blocks 25.3 -> 21.4 / 21.4 / 22.5 us; gemm_x3_kernel 22.0 /
+// 23.1 / 24.0).  Eleven, 13 and 15 would gain up to 6% at 21, 26 and 30 blocks
+// for 48 more kernels.
+int chunk_blocks(int kper) {
+    int best = 0, cost = INT_MAX;
+    for (const int ku : {16, 14, 12, 10, 9}) {
+        const int c = (kper + ku - 1) / ku * (ku + 2);
+        if (c < cost) cost = c, best = ku;
+    }
+    return best;
+}
 
 template <int FMT, int TM, int TN, int NW>
 void launch_chunks(const PairCall &c) {
-    const int c12 = chunk_cost(c.kper, 12), c14 = chunk_cost(c.kper, 14), c16 = chunk_cost(c.kper, 16);
-    if (c16 <= c14 && c16 <= c12) return launch<FMT, TM, TN, NW, 16, true>(c);
-    if (c14 <= c12) return launch<FMT, TM, TN, NW, 14, true>(c);
-    return launch<FMT, TM, TN, NW, 12, true>(c);
+    switch (chunk_blocks(c.kper)) {
+        case 16: return launch<FMT, TM, TN, NW, 16, true>(c);
+        case 14: return launch<FMT, TM, TN, NW, 14, true>(c);
+        case 12: return launch<FMT, TM, TN, NW, 12, true>(c);
+        case 10: return launch<FMT, TM, TN, NW, 10, true>(c);
+        default: return launch<FMT, TM, TN, NW, 9, true>(c);
+    }
 }
 
 template <int FMT, int TM, int TN, int NW>

@@ -24,7 +24,9 @@ def ex():
     (9, 256),       # 4 blocks, fewer features than a tile
     (200, 1664),    # 26 blocks in slices of 5 (Q8 on odd blocks, Q4 inside segments)
     (8300, 832),    # 13 blocks, 256-feature tiles, the last block short
-    (33000, 1152),  # 18 blocks, not split: two chunks
+    (33000, 1152),  # 18 blocks, not split: two chunks of nine
+    (33000, 1280),  # 20 blocks: two chunks of ten
+    (16640, 3200),  # 50 blocks in slices of 17 (Q8: chunks that start on odd blocks), the last shorter
     (16500, 2176),  # 34 blocks in slices of 12, the last shorter
     (28672, 4096),  # slices of 32: two chunks of 16
     (4096, 14336),  # slices of 28: two chunks of 14

@@ -285,12 +285,21 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_tall_kernel(const GemmArgs G,
             }
         return;
     }
+    // The tile's wide rows, a bit each: two loads by the wave (a load per row
+    // and store, and one row after another below, were 5 us of a call).
+    uint64_t wide[2] = {};
+#pragma unroll
+    for (int i = 0; i < (BM + 63) / 64; ++i) {
+        const int mi = 64 * i + lane;
+        wide[i] = __ballot(mi < BM && m0 + mi < G.n && wflags[m0 + mi] != 0);
+    }
 #pragma unroll
     for (int tm = 0; tm < TM; ++tm)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const int64_t m = m0 + tm * 16 + 4 * q + r;
-            if (m >= G.n || wflags[m]) continue;
+            const int mi = tm * 16 + 4 * q + r;
+            const int64_t m = m0 + mi;
+            if (m >= G.n || (wide[tm / 4] >> (mi & 63) & 1)) continue;
 #pragma unroll
             for (int tn = 0; tn < TN; ++tn) {
                 const int64_t j = n0 + tn * 16 + li;
@@ -301,11 +310,11 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_tall_kernel(const GemmArgs G,
             }
         }
     // this workgroup saw all of K: it recomputes its wide rows itself
-    for (int mi = 0; mi < BM && m0 + mi < G.n; ++mi) {
-        if (!wflags[m0 + mi]) continue;
-        const int64_t j = nw + tid;
-        if (j < G.rows) G.y[(m0 + mi) * G.y_stride + j] = wide_output(G, m0 + mi, j);
-    }
+    for (int i = 0; i < 2; ++i)
+        for (uint64_t left = wide[i]; left; left &= left - 1) {
+            const int64_t m = m0 + 64 * i + __builtin_ctzll(left), j = nw + tid;
+            if (j < G.rows) G.y[m * G.y_stride + j] = wide_output(G, m, j);
+        }
 }
 
 template <int FMT, int TM, int NW>

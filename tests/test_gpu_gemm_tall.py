@@ -65,3 +65,17 @@ def test_tall_tiles_match_small_tiles(ex, fmt, rows, cols, ns):
         assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), n
         got = run(ex, "srq_linear_noalloc", w, x)
         assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), n
+
+
+@pytest.mark.parametrize("fmt,rows,cols", [(srq.Q4, 32832, 256), (srq.Q8, 33000, 768)])
+@pytest.mark.parametrize("n", [66, 81, 128, 200])
+def test_unsplit_wide_rows(ex, fmt, rows, cols, n):
+    """Several rows past the FP32 limit in tiles that write y themselves, the
+    first and last of a tile and those on either side of its 64th row."""
+    rng = oracle.RNG(n)
+    w = srq.Weight.create(ex, np.resize(rng.fill_normal(1 << 18, 0.02), rows * cols).reshape(rows, cols), fmt)
+    x = rng.fill_normal(n * cols, 1.0).reshape(n, cols)
+    x[[m for m in (0, 15, 63, 64, 79, 80, n - 1) if m < n], 7] = -3e34
+    print("tall wide", fmt, rows, cols, n, flush=True)
+    got, want = run(ex, "srq_linear", w, x), small(ex, w, x)
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))

@@ -787,19 +787,39 @@ size_t gemm_scratch_bytes(int fmt, int32_t n, int64_t rows, int64_t cols) {
 }
 
 // Whether a call of n rows takes the tall tiles (gemm_tall.hip), given memory
-// for its planes.  They cost one more launch (about 4 us with its gap).
-// Q4, whose 64-row tiles here convert more per MFMA, gains from 33 rows on
-// (28672 x 4096 at 40 rows 90 -> 57 us, 512 x 512 19.7 -> 14.6 us).  Q8 gains
-// where the MFMAs outweigh the launch: 28672 x 4096 at 96 / 160 rows 101 -> 94
-// / 155 -> 115 us, 3072 x 3072 at 128 / 160 rows 21.2 -> 22.2 / 28.9 -> 28.1,
-// 5120 x 3072 at 128 / 160 rows 26.1 -> 27.6 / 36.0 -> 34.2; and not at up
-// to 64 rows of an unsplit matrix (128256 x 2048 at 40 rows 118 -> 125 us).
+// for its planes.  Q8 needs its MFMAs to outweigh the extra launch, and does
+// not gain at up to 64 rows of an unsplit matrix (128256 x 2048 at 40 rows 118
+// -> 125 us).  Otherwise the two times are estimated, in us: rounds of
+// workgroups times blocks per slice times a block, against the same of the
+// tall tile plus its split launch, which costs by activations and rows.  A block
+// (fitted so that the rule picks the faster of the two, over 1460 calls of 64 to
+// 128256 features, 256 to 14336 inputs and 33 to 1024 rows): the Q4 tile of 512
+// features 3.9; the Q8 tile of 256, two of which share a CU, 3.25, alone 2.3;
+// the tall tile of four waves 1.6, of eight 0.8 + 0.33 per 16 rows.  No call of
+// those, and one of 340 others, was then more than 3% slower than by the
+// smaller tiles (before: Q4 64 x 2048 at 1000 rows 18.0 -> 22.3 us, Q8 320 x 5120
+// at 1024 rows 33.3 -> 39.2); eleven were slower than by the tall ones (Q4 512 x
+// 2048 at 1000 rows 23.5 -> 27.5, the others by 3 to 7%).
 static bool tall_ok(const GemmPlan &p, int fmt, int32_t n, int64_t rows, int64_t cols) {
     if (!p.x3 || n <= 32 || cols % (4 * kBlock) || cols > kTallMaxCols) return false;
-    if (fmt == SRQ_Q4) return true;
-    const double macs = (double)n * (double)rows * (double)cols;
-    if (p.slices == 1 && n <= 64) return false;
-    return macs >= 3.2e9 || (n > 128 && macs >= 1.4e9);
+    if (fmt == SRQ_Q8) {
+        const double macs = (double)n * (double)rows * (double)cols;
+        if ((p.slices == 1 && n <= 64) || macs < (n > 128 ? 1.4e9 : 3.2e9)) return false;
+    }
+    auto tiles = [&](int64_t bm, int64_t bn) { return (rows + bn - 1) / bn * ((n + bm - 1) / bm) * p.slices; };
+    double small, tall;
+    if (fmt == SRQ_Q4) {
+        small = 3.9 * (double)((tiles(64, 512) + 255) / 256);
+    } else {
+        const int64_t w = tiles(64, 256), last = w % 512;
+        small = w > 1024 ? 3.25 / 512 * (double)w
+                         : 3.25 * (double)(w / 512) + (last > 256 ? 3.25 : last > 0 ? 2.3 : 0.0);
+    }
+    const TallPlan t = tall_plan(n, rows, p.slices);
+    const int64_t w = tiles(16 * t.tm, 64 * t.nw);
+    tall = t.nw == 4 ? 1.6 * (double)((w + 511) / 512) : (0.8 + 0.33 * t.tm) * (double)((w + 255) / 256);
+    const double launch = (p.slices > 1 ? 4.5 : 2.0) + 5e-6 * (double)n * (double)cols + 1.5e-3 * (double)n;
+    return (small - tall) * p.kper > launch;
 }
 
 // Layout: the wide-row flags of an unsplit call (a split one's are in its

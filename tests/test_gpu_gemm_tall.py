@@ -79,3 +79,23 @@ def test_unsplit_wide_rows(ex, fmt, rows, cols, n):
     print("tall wide", fmt, rows, cols, n, flush=True)
     got, want = run(ex, "srq_linear", w, x), small(ex, w, x)
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("fmt,rows,cols,ns", [
+    (srq.Q4, 516, 4096, (700,)),                 # 96 rows, split
+    (srq.Q4, 1030, 3328, (600, 700)),            # 112 and 128 rows, split
+    (srq.Q8, 12290, 768, (257,)),                # 96 rows, split
+    (srq.Q8, 16384, 768, (129, 200)),            # 80 and 112 rows, split
+    (srq.Q8, 4100, 1024, (800,)),                # 128 rows, split
+    (srq.Q8, 33000, 256, (200, 257, 300)),       # 80, 96 and 112 rows, not split
+    (srq.Q4, 33000, 256, (200, 257, 300)),
+])
+def test_tile_heights(ex, fmt, rows, cols, ns):
+    """Each tile height that the choice between small and tall tiles leaves in
+    use, for each format."""
+    w = srq.Weight.create(ex, np.resize(oracle.RNG(rows).fill_normal(1 << 18, 0.02), rows * cols).reshape(rows, cols), fmt)
+    for n in ns:
+        print("tall heights", fmt, rows, cols, n, flush=True)
+        x = np.resize(oracle.RNG(n).fill_normal(1 << 17, 1.0), n * cols).reshape(n, cols)
+        got, want = run(ex, "srq_linear", w, x), small(ex, w, x)
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), n

@@ -1437,9 +1437,14 @@ int launch_t(hipStream_t s, const GemvArgs &a) {
         if ((units / (blocks * kStreamWaves) + 1) * nch >= (1LL << 31))
             return fail(SRQ_EINVAL, "gemv: %lld x %lld exceeds the per-wave step limit", (long long)a.rows,
                         (long long)a.cols);
-        // One batch row of a short matrix: at most 16 units per CU.
+        // One batch row of a short matrix: at most 16 units per CU; one-row Q4
+        // units of at most 256 columns 12, past which a fourth workgroup
+        // per CU costs more than the streaming kernel (3200 .. 3968 rows 5.6 us
+        // against 6.0 here, 4096 rows 5.2 / 6.1; 3072 rows 5.5 / 5.1, and of 288
+        // columns 4096 rows 6.3 / 6.0).
         if constexpr (NB == 1 && FMT != SRQ_F32) {
-            if (a.cols <= kCoopCols && units <= 16 * cap &&
+            const int64_t per_cu = FMT == SRQ_Q4 && unit_rows_of<EPI>() == 1 && a.cols <= 256 ? 12 : 16;
+            if (a.cols <= kCoopCols && units <= per_cu * cap &&
                 ((((uintptr_t)a.x) | (NORM ? (uintptr_t)a.norm_w : 0)) & 15) == 0) {
                 launch_short<FMT, EPI, NORM>(s, a, units, nch);
                 SRQ_HIP(hipGetLastError());

@@ -21,7 +21,8 @@ def ex():
 @pytest.mark.parametrize("fmt", [srq.Q8, srq.Q4])
 @pytest.mark.parametrize("rows,cols", [(1, 32), (3, 64), (577, 576), (2048, 1024), (960, 1056), (64, 2048), (4096, 96),
                                        (4097, 160), (1000, 2080), (9, 3072),
-                                       (2050, 4064), (4096, 4096), (30, 4128)])
+                                       (2050, 4064), (4096, 4096), (30, 4128),
+                                       (3072, 256), (3073, 256), (4096, 256)])
 def test_short_gemv(ex, fmt, rows, cols):
     rng = oracle.RNG(rows + cols)
     dense = rng.fill_normal(rows * cols, 0.02).reshape(rows, cols)

@@ -199,7 +199,7 @@ def test_sample_crowded_buckets(ex, vocab, spread):
     """One far low value stretches the range, so that the other ids share a few
     first-level buckets (spread 0: one): top_k's mass comes from refined
     levels, from a sort of up to 2048 candidates or from a run of equal
-    values; chunks of one id to a full one."""
+    values; one chunk of ids to 20."""
     rng = np.random.default_rng(vocab)
     rows = 4
     logits = rng.normal(0, spread, size=(rows, vocab)).astype(np.float32)
@@ -211,6 +211,30 @@ def test_sample_crowded_buckets(ex, vocab, spread):
         got, gst = run(ex, logits, srq.Sampling(t, k, p, rp), seeds, hist)
         want, wst = oracle_rows(logits, t, k, p, rp, seeds, hist)
         assert np.array_equal(got, want), (t, k, p, got, want)
+        assert np.array_equal(gst, wst)
+
+
+@pytest.mark.parametrize("vocab", [16384, 16383])
+def test_sample_full_chunk(ex, vocab):
+    """256 rows, whose plan is one chunk a row, of the most ids a chunk holds and
+    one fewer: all ids equal, all but one in a single bucket, and spread; with
+    a penalty and blocked ids.  Counts, places and starts of a bucket then take
+    their largest values."""
+    rng = np.random.default_rng(vocab)
+    rows = 256
+    logits = rng.normal(0, 2.0, size=(rows, vocab)).astype(np.float32)
+    logits[0::3] = 1.25
+    logits[1::3] = rng.normal(0, 1e-4, size=logits[1::3].shape).astype(np.float32)
+    logits[1::3, vocab - 1] = -300.0
+    seeds = rng.integers(0, 2**63, size=rows, dtype=np.uint64)
+    hist = [list(rng.integers(0, vocab, size=7)) for _ in range(rows)]
+    blocked = np.full(rows, -1, np.int32)
+    blocked[::2] = rng.integers(0, vocab, size=rows // 2)
+    for t, k, p, rp in [(0.8, 0, 0.9, 1.1), (1.0, 40, 0.95, 1.0), (0.7, vocab - 2, 1.0, 1.2)]:
+        print("full chunk", vocab, t, k, p, rp, flush=True)
+        got, gst = run(ex, logits, srq.Sampling(t, k, p, rp), seeds, hist, blocked)
+        want, wst = oracle_rows(logits, t, k, p, rp, seeds, hist, blocked)
+        assert np.array_equal(got, want), (t, k, p)
         assert np.array_equal(gst, wst)
 
 

@@ -12,7 +12,7 @@
 // c ^ (r % 8), so that a read of one chunk of 16 rows touches every bank once.
 //
 // Measured, whole srq_linear call with its reduction, before -> now: 3072 x 576
-// at 129 rows 21.0 -> 14.1 us, 49152 x 576 at 32 / 1024 rows 47.3 -> 36.5 / 745
+// at 129 rows 21.0 -> 13.5 us, 49152 x 576 at 32 / 1024 rows 47.3 -> 36.5 / 745
 // -> 532 us (109 TFLOP/s of 157), 4096 x 2048 at 256 rows 67.8 -> 52.2 us.
 // What bounds it now: the FP32 MFMAs at many rows, the load latency of the
 // first steps and the two launches at few.

@@ -42,8 +42,6 @@ int fail(int code, const char *fmt, ...) {
     return code;
 }
 
-void clear_error() { g_err.clear(); }
-
 namespace {
 
 constexpr int kMaxDevices = 64;

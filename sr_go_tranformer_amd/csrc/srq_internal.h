@@ -47,7 +47,6 @@ __device__ __forceinline__ float nib16(uint32_t w) {
 
 // Error reporting: sets the calling thread's message and returns code.
 int fail(int code, const char *fmt, ...);
-void clear_error();
 
 #define SRQ_HIP(expr)                                                                          \
     do {                                                                                       \
